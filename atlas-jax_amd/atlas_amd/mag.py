@@ -68,25 +68,27 @@ def _swa_attention_hip(q, k, v, window, cos, sin, with_lse=False):
     return out
 
 
-def swa_attention_vjp(q, k, v, window, cos, sin, out, lse, gout):
-    """(dq, dk, dv) fp32 (B, T, H, D) of the attention core for the cotangent
-    gout of its output, on atlas_swa_bwd (the standard attention backward
-    with P recomputed from the forward's log-normalisers lse; model.py:109-129
-    differentiated)."""
+def swa_attention_vjp(q, k, v, window, cos, sin, out, lse, gout, grad_dtype=torch.float32):
+    """(dq, dk, dv) (B, T, H, D) of the attention core for the cotangent gout
+    of its output, on atlas_swa_bwd_as (the standard attention backward with
+    P recomputed from the forward's log-normalisers lse; model.py:109-129
+    differentiated).  grad_dtype: fp32, or q's dtype (the same sums rounded
+    as they are stored)."""
     lib = L.get_lib()
     B, T, H, D = q.shape
     cos = cos.float().contiguous()
     sin = sin.float().contiguous()
     gout = gout.to(out.dtype).contiguous()
-    dq = torch.empty(B, T, H, D, dtype=torch.float32, device=q.device)
+    dq = torch.empty(B, T, H, D, dtype=grad_dtype, device=q.device)
     dk = torch.empty_like(dq)
     dv = torch.empty_like(dq)
     ws_bytes = lib.atlas_swa_bwd_workspace_size(B, T, H)
     ws = torch.empty(ws_bytes, dtype=torch.uint8, device=q.device)
     sb, st, sh = q.stride(0), q.stride(1), q.stride(2)
-    L.check(lib.atlas_swa_bwd(B, T, H, D, int(window), L.ptr(q), L.ptr(k), L.ptr(v), L.ptr(out), L.ptr(gout),
-                              L.ptr(lse), sb, st, sh, L.dtype_code(q.dtype), L.ptr(cos), L.ptr(sin), L.ptr(dq),
-                              L.ptr(dk), L.ptr(dv), L.ptr(ws), ws_bytes, L.stream_ptr(q.device)))
+    L.check(lib.atlas_swa_bwd_as(B, T, H, D, int(window), L.ptr(q), L.ptr(k), L.ptr(v), L.ptr(out), L.ptr(gout),
+                                 L.ptr(lse), sb, st, sh, L.dtype_code(q.dtype), L.ptr(cos), L.ptr(sin), L.ptr(dq),
+                                 L.ptr(dk), L.ptr(dv), L.dtype_code(grad_dtype), L.ptr(ws), ws_bytes,
+                                 L.stream_ptr(q.device)))
     return dq, dk, dv
 
 
@@ -134,8 +136,8 @@ class SWAttention(torch.autograd.Function):
     @staticmethod
     def backward(ctx, gout):
         q, k, v, cos, sin, out, lse = ctx.saved_tensors
-        dq, dk, dv = swa_attention_vjp(q, k, v, ctx.window, cos, sin, out, lse, gout)
-        return dq.to(q.dtype), dk.to(k.dtype), dv.to(v.dtype), None, None, None
+        dq, dk, dv = swa_attention_vjp(q, k, v, ctx.window, cos, sin, out, lse, gout, grad_dtype=q.dtype)
+        return dq, dk, dv, None, None, None
 
     @staticmethod
     def backward_reference(q, k, v, window, cos, sin, gout):

@@ -37,6 +37,18 @@ constexpr int WAVE = 64;
 __device__ __forceinline__ int lane_id() { return threadIdx.x & (WAVE - 1); }
 __device__ __forceinline__ int wave_id() { return threadIdx.x / WAVE; }
 
+// Workgroups are dispatched to the 8 XCDs round-robin by blockIdx.x, and each
+// XCD has its own L2.  The logical block index returned here numbers the
+// blocks of one XCD consecutively, so that neighbouring logical blocks (the
+// slices of one stream, which read the same chunk operands and state) share
+// an L2.  A bijection on [0, gridDim.x) for any grid size.
+__device__ __forceinline__ int xcd_block() {
+  constexpr int kXCD = 8;
+  const int b = blockIdx.x, n = gridDim.x;
+  const int x = b % kXCD, q = n / kXCD, r = n % kXCD;
+  return x * q + (x < r ? x : r) + b / kXCD;
+}
+
 // Row of accumulator register r in lane-half h (C layout above).
 __device__ __forceinline__ constexpr int crow(int r, int h) {
   return 8 * (r >> 2) + 4 * h + (r & 3);

@@ -64,18 +64,6 @@ struct ScanArgs {
   int chunk, cur;
 };
 
-// Workgroups are dispatched to the 8 XCDs round-robin by blockIdx.x, and each
-// XCD has its own L2.  The logical block index returned here numbers the
-// blocks of one XCD consecutively, so that neighbouring logical blocks (the
-// slices of one stream, which read the same chunk operands and state) share
-// an L2.  A bijection on [0, gridDim.x) for any grid size.
-__device__ __forceinline__ int xcd_block() {
-  constexpr int kXCD = 8;
-  const int b = blockIdx.x, n = gridDim.x;
-  const int x = b % kXCD, q = n / kXCD, r = n % kXCD;
-  return x * q + (x < r ? x : r) + b / kXCD;
-}
-
 // Index of (stream, chunk)'s gate tables: the tables of a window of cw
 // consecutive chunks are held at once (slot chunk % cw).
 __device__ __forceinline__ long long chunk_table(const ScanArgs& p, int stream, int chunk) {

@@ -286,6 +286,16 @@ atlas_status atlas_swa_bwd(int32_t B, int32_t T, int32_t H, int32_t D, int32_t w
                            int32_t io_dtype, const float* cos_tab, const float* sin_tab,
                            float* dq, float* dk, float* dv,
                            void* workspace, size_t workspace_bytes, void* stream);
+/* atlas_swa_bwd with the gradients' dtype chosen: grad_dtype 0 (fp32) or
+ * io_dtype (the same fp32 sums, rounded to nearest as they are stored, for
+ * callers that would convert them). */
+atlas_status atlas_swa_bwd_as(int32_t B, int32_t T, int32_t H, int32_t D, int32_t window,
+                              const void* q, const void* k, const void* v, const void* out,
+                              const void* dout, const float* lse,
+                              int64_t stride_b, int64_t stride_t, int64_t stride_h,
+                              int32_t io_dtype, const float* cos_tab, const float* sin_tab,
+                              void* dq, void* dk, void* dv, int32_t grad_dtype,
+                              void* workspace, size_t workspace_bytes, void* stream);
 
 /* atlas_scan_fwd that also writes every chunk's start state into
  * state_trace: n_chunks = ceil(T / chunk_size) blocks of four arrays, W1

@@ -311,3 +311,58 @@ def test_swa_sweep(idx):
     e = SC.rel_l2(n(out), R.swa_core(n(q), n(k), n(v), c["window"]))
     print(f"swa sweep case {idx}: rel-L2 {e:.2e}", flush=True)
     assert e <= (2e-2 if c["dtype"] == "bf16" else 2e-3), f"case {idx} {c}: {e:.3e}"
+
+
+@pytest.mark.parametrize("dtype,tol", [("bf16", 2e-2), ("f16", 2e-3)])
+@pytest.mark.parametrize("B,T,H,window,ramp", [(8, 2500, 20, 1024, 1.0),   # 512-query workgroups
+                                               (8, 2560, 20, 4096, 12.0),  # the same, past T, rising scores
+                                               (1, 2500, 3, 1024, 12.0), (1, 513, 2, 511, 1.0),
+                                               (2, 129, 1, 128, 12.0), (1, 63, 2, 62, 1.0)])
+def test_swa_forward_tiles(dtype, tol, B, T, H, window, ramp):
+    """Both workgroup shapes of the forward at the edges of their query and
+    key tiles, with keys that grow along the sequence (ramp): the running
+    maximum then rises by more than the factor at which the accumulators are
+    rescaled.  Against the torch fp32 restatement on a few (row, head) pairs;
+    the bars are those of test_swa_kernel."""
+    torch = _torch()
+    from atlas_amd.mag import RotaryEmbedding, _rope, _swa_attention_hip, swa_attention_reference_block
+    tdt = torch.bfloat16 if dtype == "bf16" else torch.float16
+    g = torch.Generator(device="cuda").manual_seed(T + window)
+    qkv = torch.randn(B, T, 3, H, 64, device="cuda", generator=g)
+    qkv[:, :, 1] *= torch.linspace(1.0 / ramp, ramp, T, device="cuda")[None, :, None, None]
+    q, k, v = qkv.to(tdt).unbind(2)
+    cos, sin = RotaryEmbedding(64)(T)
+    out, lse = _swa_attention_hip(q, k, v, window, cos, sin, with_lse=True)
+    torch.cuda.synchronize()
+    for b, hh in {(0, 0), (B - 1, H - 1)}:
+        sl = (slice(b, b + 1), slice(None), slice(hh, hh + 1))
+        ref = swa_attention_reference_block(q[sl], k[sl], v[sl], window, cos, sin, 0, 0)
+        e = SC.rel_l2(out[sl].float().cpu().numpy(), ref.cpu().numpy())
+        qr, kr = (_rope(x[sl].float()[0, :, 0][None, :, None], cos, sin)[0, :, 0] for x in (q, k))
+        far = torch.arange(T, device="cuda")[:, None] - torch.arange(T, device="cuda")[None]
+        ref_lse = torch.logsumexp((qr @ kr.T / 8).masked_fill((far < 0) | (far > window), float("-inf")), 1)
+        # each score's fp16 operands are within 2^-11: |error| <= 2^-10 |q'||k'| / 8, typically far below
+        assert (lse[b, hh] - ref_lse).abs().max() <= 2 ** -10 * (qr.norm(dim=1) * kr.norm(dim=1).max() / 8).max()
+        print(f"swa {dtype} B{B} T{T} H{H} window {window} ({b},{hh}): rel-L2 {e:.2e}", flush=True)
+        assert e <= tol
+
+
+@pytest.mark.parametrize("dtype", ["bf16", "f16"])
+@pytest.mark.parametrize("T,window", [(129, 64), (300, 37), (64, 1000)])
+def test_swa_backward_grad_dtype(dtype, T, window):
+    """atlas_swa_bwd_as in the io dtype: the fp32 gradients rounded to nearest,
+    up to one unit in the last place (the rotation's last multiply-add may be
+    rounded once, into the io dtype, instead of twice)."""
+    torch = _torch()
+    from atlas_amd.mag import RotaryEmbedding, _swa_attention_hip, swa_attention_vjp
+    tdt = torch.bfloat16 if dtype == "bf16" else torch.float16
+    g = torch.Generator(device="cuda").manual_seed(T)
+    q, k, v = torch.randn(2, T, 3, 2, 64, device="cuda", generator=g).to(tdt).unbind(2)
+    cos, sin = RotaryEmbedding(64)(T)
+    out, lse = _swa_attention_hip(q, k, v, window, cos, sin, with_lse=True)
+    gout = torch.randn(2, T, 2, 64, device="cuda", generator=g)
+    full = swa_attention_vjp(q, k, v, window, cos, sin, out, lse, gout)
+    half = swa_attention_vjp(q, k, v, window, cos, sin, out, lse, gout, grad_dtype=tdt)
+    for a, b in zip(full, half):
+        ulp = a.abs() * torch.finfo(tdt).eps + torch.finfo(tdt).smallest_normal * torch.finfo(tdt).eps
+        assert b.dtype == tdt and bool(((a.to(tdt).float() - b.float()).abs() <= ulp).all())
