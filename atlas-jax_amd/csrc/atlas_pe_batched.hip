@@ -14,47 +14,154 @@
 #include <hip/hip_runtime.h>
 
 #include "atlas_pe.hpp"
+#include "atlas_pe_split.hpp"
 #include "atlas_scan.h"
 #include "atlas_status.hpp"
 
 namespace atlas {
 namespace {
 
-template <class M, int D, int E>
-__global__ void __launch_bounds__(256)
-pe_batched_kernel(long long n, int d1, int d2, int ns, float eps, const void* X, void* Y, int dtype) {
+// ---- one wave's matrix between global memory and C-layout tiles --------------
+// A rows x cols matrix (wide orientation, rows <= D, cols <= E) is addressed
+// through a wave-uniform pointer and 32-bit offsets, and every load is issued
+// unconditionally (out-of-range elements read element 0 and are replaced), so
+// that all loads of a matrix are in flight together; a load under a per-element
+// branch waits for the one before it (65 536 fp32 matrices of 56 x 56, 3 steps:
+// 1197 us with branches, 767 without; 3023 on fp32 operands, with branches).  Polar-Express commutes with a permutation
+// of the columns, so a wide matrix whose rows allow it gives lane c of the TJ
+// column tiles TJ consecutive columns (one load per row); a tall one (stored
+// transposed) has four consecutive rows of a column per lane by the C layout.
+enum PEPath { PE_ELEM = 0, PE_TALL4 = 1, PE_WIDEV = 2 };
+
+template <int DT>
+__device__ __forceinline__ float pe_ld1(const void* x, int o) {
+  if constexpr (DT == 0) return static_cast<const float*>(x)[o];
+  else if constexpr (DT == 1) return __uint_as_float((uint32_t)static_cast<const uint16_t*>(x)[o] << 16);
+  else return (float)static_cast<const _Float16*>(x)[o];
+}
+template <int DT>
+__device__ __forceinline__ void pe_st1(void* y, int o, float v) {
+  if constexpr (DT == 0) static_cast<float*>(y)[o] = v;
+  else if constexpr (DT == 1) static_cast<__bf16*>(y)[o] = (__bf16)v;
+  else static_cast<_Float16*>(y)[o] = (_Float16)v;
+}
+template <int N>
+struct PEVec { typedef float type __attribute__((ext_vector_type(N))); };
+
+// fp32 only for the two vector paths
+template <int D, int E, int DT, int PATH>
+__device__ __forceinline__ void pe_load(f32x16 (&X)[D / 32][E / 32], const void* x, int rows, int cols, bool tall) {
   constexpr int TI = D / 32, TJ = E / 32;
-  __shared__ __attribute__((aligned(16))) typename M::elem scr_all[4 * Scr<M>::template elems<D>()];
-  const long long mat = (long long)blockIdx.x * 4 + wave_id();
-  if (mat >= n) return;
-  typename M::elem* scr = scr_all + wave_id() * Scr<M>::template elems<D>();
   const int c = lane_id() & 31, h = lane_id() >> 5;
+  const int si = tall ? 1 : cols, sj = tall ? rows : 1;   // element strides of (i, j)
+  if constexpr (PATH == PE_TALL4) {
+#pragma unroll
+    for (int I = 0; I < TI; ++I)
+#pragma unroll
+      for (int J = 0; J < TJ; ++J)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const int i = 32 * I + 8 * q + 4 * h, j = 32 * J + c;
+          const bool ok = i < rows && j < cols;
+          const f32x4 v = *reinterpret_cast<const f32x4*>(static_cast<const float*>(x) + (ok ? j * rows + i : 0));
+#pragma unroll
+          for (int u = 0; u < 4; ++u) X[I][J][4 * q + u] = ok ? v[u] : 0.f;
+        }
+  } else if constexpr (PATH == PE_WIDEV) {
+    typedef typename PEVec<TJ>::type vec;
+#pragma unroll
+    for (int I = 0; I < TI; ++I)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int i = 32 * I + crow(r, h), j = TJ * c;
+        const bool ok = i < rows && j < cols;
+        const vec v = *reinterpret_cast<const vec*>(static_cast<const float*>(x) + (ok ? i * cols + j : 0));
+#pragma unroll
+        for (int J = 0; J < TJ; ++J) X[I][J][r] = ok ? v[J] : 0.f;
+      }
+  } else {
+#pragma unroll
+    for (int I = 0; I < TI; ++I)
+#pragma unroll
+      for (int J = 0; J < TJ; ++J)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const int i = 32 * I + crow(r, h), j = 32 * J + c;
+          const bool ok = i < rows && j < cols;
+          const float v = pe_ld1<DT>(x, ok ? i * si + j * sj : 0);
+          X[I][J][r] = ok ? v : 0.f;
+        }
+  }
+}
+// X * ps to y, laid out as pe_load reads it
+template <int D, int E, int DT, int PATH>
+__device__ __forceinline__ void pe_store(const f32x16 (&X)[D / 32][E / 32], float ps, void* y, int rows, int cols, bool tall) {
+  constexpr int TI = D / 32, TJ = E / 32;
+  // (opaque: the offsets are formed again rather than kept, spilled, across
+  // Polar-Express)
+  int lane = lane_id();
+  asm volatile("" : "+v"(lane));
+  const int c = lane & 31, h = lane >> 5;
+  const int si = tall ? 1 : cols, sj = tall ? rows : 1;
+#pragma unroll
+  for (int I = 0; I < TI; ++I) {
+    if constexpr (PATH == PE_TALL4) {
+#pragma unroll
+      for (int J = 0; J < TJ; ++J)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const int i = 32 * I + 8 * q + 4 * h, j = 32 * J + c;
+          if (i < rows && j < cols)
+            *reinterpret_cast<f32x4*>(static_cast<float*>(y) + j * rows + i) =
+                f32x4{X[I][J][4 * q] * ps, X[I][J][4 * q + 1] * ps, X[I][J][4 * q + 2] * ps, X[I][J][4 * q + 3] * ps};
+        }
+    } else if constexpr (PATH == PE_WIDEV) {
+      typedef typename PEVec<TJ>::type vec;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int i = 32 * I + crow(r, h), j = TJ * c;
+        vec v;
+#pragma unroll
+        for (int J = 0; J < TJ; ++J) v[J] = X[I][J][r] * ps;
+        if (i < rows && j < cols) *reinterpret_cast<vec*>(static_cast<float*>(y) + i * cols + j) = v;
+      }
+    } else {
+#pragma unroll
+      for (int J = 0; J < TJ; ++J)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const int i = 32 * I + crow(r, h), j = 32 * J + c;
+          if (i < rows && j < cols) pe_st1<DT>(y, i * si + j * sj, X[I][J][r] * ps);
+        }
+    }
+  }
+}
+// The widest path that a batch allows: fp32, every vector of every matrix
+// aligned (X and Y to 16 bytes; a wide matrix's rows and size, a tall one's
+// stored rows, a multiple of the vector).
+inline int pe_path(int d1, int d2, int TJ, int dtype, const void* X, const void* Y) {
+  if (dtype != 0 || ((reinterpret_cast<uintptr_t>(X) | reinterpret_cast<uintptr_t>(Y)) & 15)) return PE_ELEM;
+  if (d1 > d2) return d2 % 4 == 0 ? PE_TALL4 : PE_ELEM;
+  return TJ > 1 && d2 % TJ == 0 ? PE_WIDEV : PE_ELEM;
+}
+
+// fp32 compute mode, wide side <= 128: one wave per matrix on
+// polar_express_wave_split.
+template <int D, int E, int DT, int PATH>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
+pe_split_kernel(long long n, int d1, int d2, int ns, float eps, const void* X, void* Y) {
+  constexpr int TI = D / 32, TJ = E / 32;
+  __shared__ __attribute__((aligned(16))) _Float16 xs_all[4 * PESplit<D, E>::ELEMS];
+  const int w = __builtin_amdgcn_readfirstlane(wave_id());
+  const long long mat = (long long)blockIdx.x * 4 + w;
+  if (mat >= n) return;   // no workgroup barrier below
   const bool tall = d1 > d2;
   const int rows = tall ? d2 : d1, cols = tall ? d1 : d2;   // wide orientation
-  const long long base = mat * (long long)d1 * d2;
+  const long long base = mat * (long long)d1 * d2 * (DT == 0 ? 4 : 2);
   f32x16 Xr[TI][TJ];
-#pragma unroll
-  for (int I = 0; I < TI; ++I)
-#pragma unroll
-    for (int J = 0; J < TJ; ++J)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int i = 32 * I + crow(r, h), j = 32 * J + c;   // (row, col) of the wide form
-        float v = 0.f;
-        if (i < rows && j < cols) v = load_any(X, base + (tall ? (long long)j * d2 + i : (long long)i * d2 + j), dtype);
-        Xr[I][J][r] = v;
-      }
-  polar_express_wave<M, D, E>(Xr, ns, eps, scr);
-#pragma unroll
-  for (int I = 0; I < TI; ++I)
-#pragma unroll
-    for (int J = 0; J < TJ; ++J)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int i = 32 * I + crow(r, h), j = 32 * J + c;
-        if (i < rows && j < cols)
-          store_any(Y, base + (tall ? (long long)j * d2 + i : (long long)i * d2 + j), dtype, Xr[I][J][r]);
-      }
+  pe_load<D, E, DT, PATH>(Xr, static_cast<const char*>(X) + base, rows, cols, tall);
+  const float ps = polar_express_wave_split<D, E>(Xr, ns, eps, xs_all + w * PESplit<D, E>::ELEMS);
+  pe_store<D, E, DT, PATH>(Xr, ps, static_cast<char*>(Y) + base, rows, cols, tall);
 }
 
 // fp16 operands, wide side <= 128: the scan's own Polar-Express
@@ -410,12 +517,18 @@ atlas_status launch_pair(long long n, int d1, int d2, int ns, float eps, const v
   return e == hipSuccess ? ATLAS_OK : fail_hip(e, "pe_batched launch");
 }
 
-template <class M, int D, int E>
-atlas_status launch(long long n, int d1, int d2, int ns, float eps, const void* X, void* Y, int dtype,
-                    hipStream_t st) {
+template <int D, int E>
+atlas_status launch_split(long long n, int d1, int d2, int ns, float eps, const void* X, void* Y, int dtype,
+                          hipStream_t st) {
   const long long blocks = (n + 3) / 4;
-  hipLaunchKernelGGL((pe_batched_kernel<M, D, E>), dim3((unsigned)blocks), dim3(256), 0, st, n, d1, d2, ns, eps, X,
-                     Y, dtype);
+  const int path = pe_path(d1, d2, E / 32, dtype, X, Y);
+  using K = void (*)(long long, int, int, int, float, const void*, void*);
+  auto go = [&](K k) { hipLaunchKernelGGL(k, dim3((unsigned)blocks), dim3(256), 0, st, n, d1, d2, ns, eps, X, Y); };
+  if (dtype == 1) go(pe_split_kernel<D, E, 1, PE_ELEM>);
+  else if (dtype == 2) go(pe_split_kernel<D, E, 2, PE_ELEM>);
+  else if (path == PE_TALL4) go(pe_split_kernel<D, E, 0, PE_TALL4>);
+  else if (path == PE_WIDEV) go(pe_split_kernel<D, E, 0, (E > 32) ? PE_WIDEV : PE_ELEM>);
+  else go(pe_split_kernel<D, E, 0, PE_ELEM>);
   const hipError_t e = hipGetLastError();
   return e == hipSuccess ? ATLAS_OK : fail_hip(e, "pe_batched launch");
 }
@@ -457,11 +570,11 @@ atlas_status dispatch(long long n, int d1, int d2, int ns, float eps, const void
     if (D == 64 && E == 64) return launch_t<64, 64>(n, d1, d2, ns, eps, X, Y, dtype, st);
     return launch_t<64, 128>(n, d1, d2, ns, eps, X, Y, dtype, st);
   }
-  if (D == 32 && E == 32) return launch<M, 32, 32>(n, d1, d2, ns, eps, X, Y, dtype, st);
-  if (D == 32 && E == 64) return launch<M, 32, 64>(n, d1, d2, ns, eps, X, Y, dtype, st);
-  if (D == 32 && E == 128) return launch<M, 32, 128>(n, d1, d2, ns, eps, X, Y, dtype, st);
-  if (D == 64 && E == 64) return launch<M, 64, 64>(n, d1, d2, ns, eps, X, Y, dtype, st);
-  return launch<M, 64, 128>(n, d1, d2, ns, eps, X, Y, dtype, st);
+  if (D == 32 && E == 32) return launch_split<32, 32>(n, d1, d2, ns, eps, X, Y, dtype, st);
+  if (D == 32 && E == 64) return launch_split<32, 64>(n, d1, d2, ns, eps, X, Y, dtype, st);
+  if (D == 32 && E == 128) return launch_split<32, 128>(n, d1, d2, ns, eps, X, Y, dtype, st);
+  if (D == 64 && E == 64) return launch_split<64, 64>(n, d1, d2, ns, eps, X, Y, dtype, st);
+  return launch_split<64, 128>(n, d1, d2, ns, eps, X, Y, dtype, st);
 }
 
 }  // namespace

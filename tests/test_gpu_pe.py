@@ -232,3 +232,40 @@ def test_pe_sweep(idx):
         bound = max(2e-2, 3.0 * SC.rel_l2(_pe_rounded("f16")(X, c["ns"]), ref))
     print(f"pe sweep case {idx}: rel-L2 {err:.2e} (bound {bound:.2e})", flush=True)
     assert err <= bound, f"case {idx} {c}: {err:.3e} > {bound:.3e}"
+
+
+@pytest.mark.parametrize("d1,d2", [(64, 64), (64, 128), (128, 64), (63, 64), (56, 56), (33, 127), (32, 32), (31, 100),
+                                   (100, 12), (30, 62), (1, 1)])
+@pytest.mark.parametrize("kind", ["random", "decaying", "tiny"])
+def test_pe_fp32_split_accuracy(d1, d2, kind):
+    """fp32 mode on operands held as two fp16 numbers: at every load path (16-
+    and 4-byte aligned buffers, whole and partial tiles) the error against
+    float64 stays within twice that of the same iteration in fp32 torch (its
+    rounding per product is 2^-24; the two halves' 2^-23)."""
+    torch = _torch()
+    from atlas_amd import POLAR_EXPRESS_COEFFS, polar_express
+    g = torch.Generator(device="cuda").manual_seed(d1 * 257 + d2)
+    n, steps = 37, 5
+    X = torch.randn(n, d1, d2, device="cuda", generator=g)
+    if kind != "random":   # a momentum: rank-one terms that halve from token to token
+        u, v = torch.randn(n, 64, d1, device="cuda", generator=g), torch.randn(n, 64, d2, device="cuda", generator=g)
+        w = 0.5 ** torch.arange(64.0, device="cuda")[None, :, None]
+        X = (w * u).mT.contiguous() @ v * (1e-3 if kind == "decaying" else 1e-9)
+
+    def plain(x):
+        x = x / (torch.sqrt((x * x).sum((-2, -1), keepdim=True) + 1e-12) * 1.01 + 1e-6)
+        for a, b, c in POLAR_EXPRESS_COEFFS[:steps]:
+            A = x @ x.mT.contiguous() if d1 <= d2 else x.mT.contiguous() @ x
+            B = b * A + c * (A @ A)
+            x = a * x + (B @ x if d1 <= d2 else x @ B)
+        return x
+
+    ref = plain(X.double())
+    rel = lambda y: float((y.double() - ref).norm() / ref.norm())  # noqa: E731
+    # (at least 2^-23 for each operand of the 3 products of 5 steps, which a few scalars alone can show)
+    bar = max(2 * rel(plain(X)), 2 * 3 * steps * 2.0 ** -24)
+    odd = torch.empty(X.numel() + 1, device="cuda")[1:].view(n, d1, d2).copy_(X)
+    for x in (X, odd):
+        e = rel(polar_express(x, steps, precision="f32"))
+        print(f"split PE {d1}x{d2} {kind}: {e:.2e} (bar {bar:.2e})", flush=True)
+        assert e <= bar
