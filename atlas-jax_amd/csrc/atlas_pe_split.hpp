@@ -21,6 +21,11 @@ namespace atlas {
 struct SFrag {
   f16x8 hi, lo;
 };
+__device__ __forceinline__ int opaque_lane() {
+  int l = lane_id();
+  asm volatile("" : "+v"(l));
+  return l;
+}
 // (The pair is opaque between the conversion and the subtraction: formed
 // twice, by two different instructions, a hi on a rounding boundary could
 // differ from the one that lo completes.)
@@ -113,8 +118,11 @@ struct PESplit {
     *reinterpret_cast<f16x4*>(p + BLOCK) = lo;
   }
   // column block J of X: lane (c, h) writes d = 32I + 8q + 4h + 0..3 of row c
-  __device__ __forceinline__ static void put_block(const f32x16 (&X)[TI][TJ], int J, float s, _Float16* xs) {
-    const int c = lane_id() & 31, h = lane_id() >> 5;
+  // (ln: the lane, which a caller may pass through an opaque value so that the
+  // offsets are formed where they are used instead of held across its loops)
+  __device__ __forceinline__ static void put_block(const f32x16 (&X)[TI][TJ], int J, float s, _Float16* xs,
+                                                   int ln = lane_id()) {
+    const int c = ln & 31, h = ln >> 5;
 #pragma unroll
     for (int I = 0; I < TI; ++I)
 #pragma unroll
@@ -125,19 +133,19 @@ struct PESplit {
     return f16x8{a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
   }
   // Gram fragment: lane l holds X[32I + l % 32][columns 16 kb + 8 (l / 32) + v of the block]
-  __device__ __forceinline__ static SFrag get(const _Float16* xs, int I, int kb) {
-    const int l = lane_id(), j = l & 15, r = 16 * kb + 8 * (l >> 5) + (j >> 2), u = 8 * I + 4 * ((l >> 4) & 1) + (j & 3);
+  __device__ __forceinline__ static SFrag get(const _Float16* xs, int I, int kb, int l = lane_id()) {
+    const int j = l & 15, r = 16 * kb + 8 * (l >> 5) + (j >> 2), u = 8 * I + 4 * ((l >> 4) & 1) + (j & 3);
     const _Float16 *p = xs + at(r, u), *p4 = xs + at(r + 4, u);
     return {tr2(p, p4), tr2(p + BLOCK, p4 + BLOCK)};
   }
   // A 32 x 32 C-layout tile times s, transposed: fragments with k in C-layout order
-  __device__ __forceinline__ static void put_tile(const f32x16& t, float s, _Float16* xs) {
-    const int c = lane_id() & 31, h = lane_id() >> 5;
+  __device__ __forceinline__ static void put_tile(const f32x16& t, float s, _Float16* xs, int ln = lane_id()) {
+    const int c = ln & 31, h = ln >> 5;
 #pragma unroll
     for (int q = 0; q < 4; ++q) put4(t, q, s, xs + at(c, 2 * q + h));
   }
-  __device__ __forceinline__ static SFrag get_tile(const _Float16* xs, int kb) {
-    const int l = lane_id(), j = l & 15, r = 16 * kb + 4 * (l >> 5) + (j >> 2), u = 4 * ((l >> 4) & 1) + (j & 3);
+  __device__ __forceinline__ static SFrag get_tile(const _Float16* xs, int kb, int l = lane_id()) {
+    const int j = l & 15, r = 16 * kb + 4 * (l >> 5) + (j >> 2), u = 4 * ((l >> 4) & 1) + (j & 3);
     const _Float16 *p = xs + at(r, u), *p8 = xs + at(r + 8, u);
     return {tr2(p, p8), tr2(p + BLOCK, p8 + BLOCK)};
   }

@@ -43,6 +43,7 @@
 
 #include "atlas_common.hpp"
 #include "atlas_pe.hpp"
+#include "atlas_pe_vjp_split.hpp"
 #include "atlas_scan.h"
 #include "atlas_status.hpp"
 
@@ -63,7 +64,7 @@ constexpr int BT = 256;           // threads per block
 constexpr int NWV = BT / WAVE;    // waves per block
 constexpr int EPT = 4;            // state elements per thread in the element-wise scans
 constexpr int EBLK = BT * EPT;    // state elements per block
-constexpr int VJP_GRID = 256;     // persistent workgroups of the fp32 Polar-Express VJP (one per CU)
+constexpr int VJP_GRID = 256;     // CUs the fp32 Polar-Express VJP's persistent workgroups and scratch are sized for
 constexpr int VJPW_GRID = 256;    // persistent workgroups of the per-wave fp16 VJP (one per CU)
 
 struct BwdArgs {
@@ -737,213 +738,20 @@ __global__ void gate_grad_kernel(BwdArgs a, long long pchunk, long long cbase) {
   a.det[gi] = se;
 }
 
-// ---- Polar-Express VJP per matrix ----------------------------------------
-// One workgroup per matrix at a time (persistent over the batch).  The matrix
-// X (D x E, E >= D; `tall` = stored transposed, E x D) and its cotangent live
-// in LDS as fp32 (for 64 x 256, where they and the four D x D products would
-// need 198 KiB, in the workgroup's global scratch instead: all waves of a
-// workgroup share one CU's L1, and every exchange through them is ordered by
-// a workgroup barrier); the iterates Y_0 .. Y_{ns-2} of the forward
-// recompute are kept in a per-workgroup global scratch area.  Products use fp32 MFMA
-// (v_mfma_f32_32x32x2f32) with operands read from LDS.  VJP of one step
-// Y' = a Y + (b A + c A^2) Y, A = Y Y^T, for the cotangent G of Y':
-//   G_Y = a G + B G + (b Gs + c (Gs A + A Gs)) Y,  Gs = G Y^T + Y G^T;
-// then the normalisation's VJP: dX = G / nrm - (<G, X> 1.01 / (nrm^2 n)) X.
-
-// acc += sum_k A(r, k) B(k, c) for tile (I, J); A(r, k) = Ap[r*ars + k*aks],
-// B(k, c) = Bp[k*bks + c*bcs].
-__device__ __forceinline__ f32x16 tile_mma(f32x16 acc, int I, int J, int K, const float* Ap, int ars, int aks,
-                                           const float* Bp, int bks, int bcs) {
-  const int c = lane_id() & 31, hf = lane_id() >> 5;
-  const float* ap = Ap + (32 * I + c) * ars + hf * aks;
-  const float* bp = Bp + hf * bks + (32 * J + c) * bcs;
-#pragma unroll 8
-  for (int k0 = 0; k0 < K; k0 += 2)
-    acc = __builtin_amdgcn_mfma_f32_32x32x2f32(ap[k0 * aks], bp[k0 * bks], acc, 0, 0, 0);
-  return acc;
-}
-
-template <int D, int E>
-struct VjpLds {
-  static constexpr int LE = E + 1, LD = D + 1;   // odd row strides: conflict-free column reads
-  // the iterate Y and the cotangent Gb in LDS (else in the global scratch)
-  static constexpr bool YG_LDS = (2 * D * LE + 4 * D * LD + 2 * NWV) * sizeof(float) <= 160 * 1024;
-  static constexpr int bytes() { return ((YG_LDS ? 2 * D * LE : 0) + 4 * D * LD + 2 * NWV) * (int)sizeof(float); }
-  // per-workgroup global scratch (floats): the iterates, and Y and Gb when not in LDS
-  static constexpr size_t scratch_floats(int ns) {
-    return (size_t)(ns > 1 ? ns - 1 : 1) * D * E + (YG_LDS ? 0 : (size_t)2 * D * LE);
-  }
-};
-
-template <int D, int E>
-__global__ void __launch_bounds__(BT) pe_vjp_kernel(long long n, int ns, int tall, const float* X, float* G,
-                                                    float* scratch) {
-  using LY = VjpLds<D, E>;
-  constexpr int LE = LY::LE, LD = LY::LD;
-  constexpr int TN = (D / 32) * (E / 32), TA = (D / 32) * (D / 32);
-  constexpr int TNW = (TN + NWV - 1) / NWV, TAW = (TA + NWV - 1) / NWV;
-  extern __shared__ __attribute__((aligned(16))) float sm[];
-  float* scr = scratch + (long long)blockIdx.x * LY::scratch_floats(ns);
-  float* Y = LY::YG_LDS ? sm : scr + (size_t)(ns > 1 ? ns - 1 : 1) * D * E;
-  float* Gb = Y + D * LE;
-  float* A = LY::YG_LDS ? Gb + D * LE : sm;
-  float* Bm = A + D * LD;
-  float* Gs = Bm + D * LD;
-  float* T1 = Gs + D * LD;
-  float* red = T1 + D * LD;
-  const int tid = threadIdx.x, wv = wave_id(), c = lane_id() & 31, hf = lane_id() >> 5;
-
-  auto at = [&](long long base, int d, int e) -> long long {
-    return base + (tall ? (long long)e * D + d : (long long)d * E + e);
-  };
-  // A = Y Y^T into A, then Bm = b A + c A^2 (T1 scratch)
-  auto gram_b = [&](float b, float cc) {
-    for (int tl = wv; tl < TA; tl += NWV) {
-      const int I = tl / (D / 32), J = tl % (D / 32);
-      const f32x16 acc = tile_mma(zero16(), I, J, E, Y, LE, 1, Y, 1, LE);
-#pragma unroll
-      for (int r = 0; r < 16; ++r) A[(32 * I + crow(r, hf)) * LD + 32 * J + c] = acc[r];
-    }
-    __syncthreads();
-    for (int tl = wv; tl < TA; tl += NWV) {
-      const int I = tl / (D / 32), J = tl % (D / 32);
-      const f32x16 acc = tile_mma(zero16(), I, J, D, A, LD, 1, A, LD, 1);
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int o = (32 * I + crow(r, hf)) * LD + 32 * J + c;
-        Bm[o] = b * A[o] + cc * acc[r];
-      }
-    }
-    __syncthreads();
-  };
-
-  for (long long mi = blockIdx.x; mi < n; mi += gridDim.x) {
-    const long long base = mi * D * E;
-    float ss = 0.f;
-    for (int i = tid; i < D * E; i += BT) {
-      const int d = i / E, e = i % E;
-      const float x = X[at(base, d, e)];
-      Y[d * LE + e] = x;
-      ss = fmaf(x, x, ss);
-    }
-    const float nn = sqrtf(block_sum(ss, red, 0) + 1e-12f);
-    const float nrm = nn * 1.01f + 1e-6f;
-    for (int i = tid; i < D * E; i += BT) {
-      const int d = i / E, e = i % E;
-      Y[d * LE + e] = Y[d * LE + e] / nrm;
-    }
-    __syncthreads();
-    // forward recompute: Y_0 .. Y_{ns-1}; Y_0 .. Y_{ns-2} to scratch
-    for (int k = 0; k + 1 < ns; ++k) {
-      for (int i = tid; i < D * E; i += BT) scr[(long long)k * D * E + i] = Y[(i / E) * LE + i % E];
-      gram_b(kPE[k][1], kPE[k][2]);
-      f32x16 acc[TNW];
-#pragma unroll
-      for (int q = 0; q < TNW; ++q) {
-        const int tl = wv + q * NWV;
-        if (tl < TN) acc[q] = tile_mma(zero16(), tl / (E / 32), tl % (E / 32), D, Bm, LD, 1, Y, LE, 1);
-      }
-      __syncthreads();
-      const float ak = kPE[k][0];
-#pragma unroll
-      for (int q = 0; q < TNW; ++q) {
-        const int tl = wv + q * NWV;
-        if (tl >= TN) continue;
-        const int I = tl / (E / 32), J = tl % (E / 32);
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int o = (32 * I + crow(r, hf)) * LE + 32 * J + c;
-          Y[o] = ak * Y[o] + acc[q][r];
-        }
-      }
-      __syncthreads();
-    }
-    // backward through the steps
-    for (int i = tid; i < D * E; i += BT) Gb[(i / E) * LE + i % E] = G[at(base, i / E, i % E)];
-    __syncthreads();
-    for (int k = ns - 1; k >= 0; --k) {
-      if (k + 1 < ns) {
-        for (int i = tid; i < D * E; i += BT) Y[(i / E) * LE + i % E] = scr[(long long)k * D * E + i];
-        __syncthreads();
-      }
-      const float ak = kPE[k][0], bk = kPE[k][1], ck = kPE[k][2];
-      gram_b(bk, ck);
-      // Gh = Gb Y^T -> T1, then Gs = Gh + Gh^T
-      for (int tl = wv; tl < TA; tl += NWV) {
-        const int I = tl / (D / 32), J = tl % (D / 32);
-        const f32x16 acc = tile_mma(zero16(), I, J, E, Gb, LE, 1, Y, 1, LE);
-#pragma unroll
-        for (int r = 0; r < 16; ++r) T1[(32 * I + crow(r, hf)) * LD + 32 * J + c] = acc[r];
-      }
-      __syncthreads();
-      for (int i = tid; i < D * D; i += BT) {
-        const int r = i / D, q = i % D;
-        Gs[r * LD + q] = T1[r * LD + q] + T1[q * LD + r];
-      }
-      __syncthreads();
-      // T1 = Gs A + A Gs, then Gs <- b Gs + c T1
-      for (int tl = wv; tl < TA; tl += NWV) {
-        const int I = tl / (D / 32), J = tl % (D / 32);
-        f32x16 acc = tile_mma(zero16(), I, J, D, Gs, LD, 1, A, LD, 1);
-        acc = tile_mma(acc, I, J, D, A, LD, 1, Gs, LD, 1);
-#pragma unroll
-        for (int r = 0; r < 16; ++r) T1[(32 * I + crow(r, hf)) * LD + 32 * J + c] = acc[r];
-      }
-      __syncthreads();
-      for (int i = tid; i < D * D; i += BT) {
-        const int o = (i / D) * LD + i % D;
-        Gs[o] = bk * Gs[o] + ck * T1[o];
-      }
-      __syncthreads();
-      // Gb <- a Gb + Bm Gb + Gs Y
-      f32x16 acc[TNW];
-#pragma unroll
-      for (int q = 0; q < TNW; ++q) {
-        const int tl = wv + q * NWV;
-        if (tl >= TN) continue;
-        const int I = tl / (E / 32), J = tl % (E / 32);
-        acc[q] = tile_mma(zero16(), I, J, D, Bm, LD, 1, Gb, LE, 1);
-        acc[q] = tile_mma(acc[q], I, J, D, Gs, LD, 1, Y, LE, 1);
-      }
-      __syncthreads();
-#pragma unroll
-      for (int q = 0; q < TNW; ++q) {
-        const int tl = wv + q * NWV;
-        if (tl >= TN) continue;
-        const int I = tl / (E / 32), J = tl % (E / 32);
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int o = (32 * I + crow(r, hf)) * LE + 32 * J + c;
-          Gb[o] = ak * Gb[o] + acc[q][r];
-        }
-      }
-      __syncthreads();
-    }
-    // normalisation
-    float dot = 0.f;
-    for (int i = tid; i < D * E; i += BT) dot = fmaf(Gb[(i / E) * LE + i % E], X[at(base, i / E, i % E)], dot);
-    const float coef = block_sum(dot, red, 1) * 1.01f / (nrm * nrm * nn);
-    for (int i = tid; i < D * E; i += BT) {
-      const long long o = at(base, i / E, i % E);
-      G[o] = Gb[(i / E) * LE + i % E] / nrm - coef * X[o];
-    }
-    __syncthreads();
-  }
-  (void)TAW;
-}
-
 template <int D, int E>
 atlas_status launch_vjp(long long n, int ns, int tall, const float* X, float* G, float* scratch, hipStream_t st) {
-  const int bytes = VjpLds<D, E>::bytes();
+  using V = VjpSplit<D, E>;
+  const int bytes = (int)V::bytes();
   static bool attr_set = false;   // the attribute is per function, not per device
   if (!attr_set) {
-    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&pe_vjp_kernel<D, E>),
+    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&pe_vjp_split_kernel<D, E>),
                                              hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
     if (e != hipSuccess) return fail_hip(e, "pe_vjp shared-memory attribute");
     attr_set = true;
   }
-  const long long grid = std::min<long long>(n, VJP_GRID);
-  hipLaunchKernelGGL((pe_vjp_kernel<D, E>), dim3((unsigned)grid), dim3(BT), bytes, st, n, ns, tall, X, G, scratch);
+  // the scratch holds VJP_GRID x (ns - 1) iterates: enough for PER_CU (at most 2) workgroups per slot
+  const long long grid = std::min<long long>(n, (long long)V::PER_CU * VJP_GRID);
+  hipLaunchKernelGGL((pe_vjp_split_kernel<D, E>), dim3((unsigned)grid), dim3(256), bytes, st, n, ns, tall, X, G, scratch);
   const hipError_t e = hipGetLastError();
   return e == hipSuccess ? ATLAS_OK : fail_hip(e, "pe_vjp launch");
 }
@@ -1953,9 +1761,7 @@ atlas_status pe_vjp_both(long long n, int D, int E, int ns, const float* X0, flo
 
 size_t vjp_scratch_floats(int D, int E, int ns) {
   // the fp32 VJP's per-workgroup scratch (the fp16 VJP needs none)
-  size_t f32 = (size_t)(ns > 1 ? ns - 1 : 1) * D * E;
-  if (D == 64 && E == 256) f32 = VjpLds<64, 256>::scratch_floats(ns);
-  return (size_t)VJP_GRID * f32;
+  return (size_t)VJP_GRID * (ns > 1 ? ns - 1 : 1) * D * E;
 }
 
 // Shapes the backward is compiled for.

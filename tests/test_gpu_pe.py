@@ -269,3 +269,37 @@ def test_pe_fp32_split_accuracy(d1, d2, kind):
         e = rel(polar_express(x, steps, precision="f32"))
         print(f"split PE {d1}x{d2} {kind}: {e:.2e} (bar {bar:.2e})", flush=True)
         assert e <= bar
+
+
+@pytest.mark.parametrize("d1,d2", [(32, 32), (64, 32), (32, 128), (64, 64), (64, 128), (128, 64), (64, 256), (256, 64)])
+@pytest.mark.parametrize("steps,n", [(0, 3), (1, 3), (2, 3), (3, 3), (4, 3), (5, 3), (5, 600)])
+@pytest.mark.parametrize("gscale", [1e-20, 1.0, 1e15])
+def test_pe_vjp_f32_split_accuracy(d1, d2, steps, n, gscale):
+    """fp32 VJP on operands held as two fp16 numbers: every number of steps
+    (the iterates come from registers, scratch or X), more matrices than
+    resident workgroups, cotangents of any size, against float64 autograd;
+    within twice the error of the same derivative by fp32 autograd, and at
+    least 2^-23 for each operand of the 8 products of a step."""
+    torch = _torch()
+    from atlas_amd import POLAR_EXPRESS_COEFFS
+    from atlas_amd.autograd import polar_express_vjp
+    g = torch.Generator(device="cuda").manual_seed(d1 * 257 + d2 + steps)
+    X = torch.randn(n, d1, d2, device="cuda", generator=g) * 1e-3
+    C = torch.randn(n, d1, d2, device="cuda", generator=g) * gscale
+
+    def grad(x, c):
+        x = x.clone().requires_grad_(True)
+        y = x / (torch.sqrt((x * x).sum((-2, -1), keepdim=True) + 1e-12) * 1.01 + 1e-6)
+        for a, b, cc in POLAR_EXPRESS_COEFFS[:steps]:
+            A = y @ y.mT.contiguous() if d1 <= d2 else y.mT.contiguous() @ y
+            B = b * A + cc * (A @ A)
+            y = a * y + (B @ y if d1 <= d2 else y @ B)
+        return torch.autograd.grad(y, x, c)[0]
+
+    sel = torch.arange(n)[-64:]
+    ref = grad(X[sel].double(), C[sel].double())
+    rel = lambda y: float((y.double() - ref).norm() / ref.norm())  # noqa: E731
+    bar = max(2 * rel(grad(X[sel], C[sel])), 2 * 8 * max(steps, 1) * 2.0 ** -24)
+    e = rel(polar_express_vjp(X, C, steps)[sel])
+    print(f"split VJP {d1}x{d2} ns{steps} n={n} G {gscale:g}: {e:.2e} (bar {bar:.2e})", flush=True)
+    assert e <= bar
