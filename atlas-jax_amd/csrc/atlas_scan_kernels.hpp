@@ -26,6 +26,7 @@
 
 #include "atlas_common.hpp"
 #include "atlas_pe.hpp"
+#include "atlas_pe_split.hpp"
 
 namespace atlas {
 
@@ -592,6 +593,7 @@ phase_kernel(ScanArgs p) {
   using elem = typename M::elem;
   using frag = typename M::frag;
   using LY = PhaseLayout<M, D, E>;
+  static_assert(sizeof(elem) == 4, "fp32 mode (the fp16 mode runs phase16_kernel and phase_wide_kernel)");
   extern __shared__ __attribute__((aligned(16))) char smem[];
   const LY L(p.cs);
 
@@ -901,7 +903,16 @@ phase_kernel(ScanArgs p) {
       }
     }
 
-    polar_express_wave<M, D, E>(X, p.ns, 1e-12f, scr);
+    // (on operands as two fp16 numbers, its staging in the scratch: at 64 x 128 a
+    // launch of 256 workgroups with four tokens per wave takes half the time of
+    // the step on fp32 MFMA)
+    {
+      const float ps = polar_express_wave_split<D, E>(X, p.ns, 1e-12f, reinterpret_cast<_Float16*>(scr));
+#pragma unroll
+      for (int I = 0; I < TI; ++I)
+#pragma unroll
+        for (int J = 0; J < TJ; ++J) X[I][J] *= ps;
+    }
 
     // memory-scan partial L += a(s->end_j) P and the slice read-out partial.
     const float aend = ass[sl * ts + ts - 1];
@@ -929,16 +940,12 @@ phase_kernel(ScanArgs p) {
         __syncthreads();
       }
     } else {
-      typename M::afrag aid[KPT];
-#pragma unroll
-      for (int kb = 0; kb < KPT; ++kb) aid[kb] = M::a_identity(kb, c, h, aend);
 #pragma unroll
       for (int I = 0; I < (LSH ? 1 : TI); ++I)
 #pragma unroll
         for (int J = 0; J < (LSH ? 1 : TJ); ++J)
 #pragma unroll
-          for (int kb = 0; kb < KPT; ++kb)
-            Lacc[I][J] = M::amma(aid[kb], M::a_from_c(X[I][J], kb), Lacc[I][J]);
+          for (int r = 0; r < 16; ++r) Lacc[I][J][r] = fmaf(aend, X[I][J][r], Lacc[I][J][r]);
     }
     if (MAT == 2) {
       // hloc[e][t'] += sum_d P2[e][d] q_t'[d] w(t')  (X tiles as A operand = P2 rows e)
