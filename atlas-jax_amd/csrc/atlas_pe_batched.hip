@@ -9,9 +9,11 @@
 // zero rows/columns stay zero through every Newton-Schulz step, so padding
 // does not change the result.  Wide sides of 129..256 are split over a pair
 // of waves (128 columns each, the Gram summed through LDS).  Short sides of
-// 65..128 run on a workgroup of eight waves per matrix (pe_wg_kernel, fp32
-// operands).
+// 65..128 run on a workgroup of six or eight waves per matrix (pe_wg_kernel,
+// fp32 accuracy).
 #include <hip/hip_runtime.h>
+
+#include <algorithm>
 
 #include "atlas_pe.hpp"
 #include "atlas_pe_split.hpp"
@@ -331,56 +333,117 @@ pe_pair_kernel(long long n, int d1, int d2, int ns, float eps, const void* X, vo
       }
 }
 
-// One workgroup of eight waves per matrix whose short side is 65..128 (TI =
-// 3 or 4 row tiles of 32; long side <= 256), fp32 matrix-core operands in
-// either compute mode.  The iterate X (wide orientation, zero-padded to TI x
-// 32 rows and whole 32-column blocks) is held in registers as C-layout tiles,
-// column block J by wave J.  Per Newton-Schulz step:
-//   Gram  G = X X^T: the column blocks are staged in LDS one at a time (fp32
-//         rows d, double buffered) and every wave accumulates its own tiles
-//         of G (tile t = wave + 8q) over all blocks;
-//   B     = b G + c G^2 from G in LDS (each wave its own tiles), written back
-//         over G once every wave has read it;
-//   X     <- a X + B X for the wave's column block, B from LDS.
-// Every sum has a fixed order (bitwise reproducible).  LDS: two staging
-// blocks (DP x 33 floats) and G/B (DP x (DP + 1) floats), at most 100 KiB.
-template <int TI>
+// One workgroup of NW waves per matrix whose short side is 65..128 (TI = 3 or
+// 4 row tiles of 32; long side <= 32 NW <= 256), in fp32 accuracy in either
+// compute mode: operands as two fp16 numbers (atlas_pe_split.hpp).  The iterate
+// X (wide orientation, zero-padded to 32 TI rows and whole 32-column blocks) is
+// held in registers as fp32 C-layout tiles, column block J by wave J.  Per
+// Newton-Schulz step, with barriers between:
+//   X's blocks staged in LDS as split rows, all at once;
+//   Gram: each wave forms its upper tiles of G = X X^T over all blocks;
+//   G shared as operand fragments (every lane writes the 16 bytes that the
+//         same lane of the other waves reads; a lower tile is its mirror
+//         transposed through its own slot), laid over the staged blocks;
+//   B     = b G + c G^2, the same tiles, shared the same way;
+//   X     <- a X + B X for the wave's column block.
+// Every sum has a fixed order (bitwise reproducible).  2 048 matrices of 96 x
+// 192, 5 steps: 356 us (1019 us on fp32 operands, staged a block at a time
+// with all nine Gram tiles).
+template <int TI, int NW>
 struct PEWg {
-  static constexpr int NWG = 8;
   static constexpr int DP = 32 * TI;
-  static constexpr int SS = 33;                 // staging row stride (floats)
-  static constexpr int GS = DP + 1;             // G/B row stride (floats)
-  static constexpr int NT = (TI * TI + NWG - 1) / NWG;
-  static constexpr size_t lds_bytes() { return (size_t)(2 * DP * SS + DP * GS + NWG) * sizeof(float); }
+  static constexpr int NT = TI * (TI + 1) / 2;        // upper tiles
+  static constexpr int NQ = (NT + NW - 1) / NW;       // of a wave, at most
+  static constexpr int BLK = PESplit<DP, 32>::ELEMS;  // halves of a staged block
+  static constexpr int FR = TI * TI * 2 * 2 * 512;    // halves of G or B as fragments
+  static size_t lds_bytes(int nj) { return (size_t)std::max(nj * BLK, 2 * FR) * 2 + NW * sizeof(float); }
+  // (I, I2 >= I) of upper tile t, row by row
+  __device__ __forceinline__ static void tile(int t, int& I, int& I2) {
+    I = 0;
+    int n = TI;
+    while (t >= n) {
+      t -= n;
+      --n;
+      ++I;
+    }
+    I2 = I + t;
+  }
 };
 
-template <int TI>
-__global__ void __launch_bounds__(512)
-pe_wg_kernel(long long n, int d1, int d2, int ns, float eps, const void* X, void* Y, int dtype) {
-  using W = PEWg<TI>;
-  using M = ModeF32;
-  constexpr int DP = W::DP, SS = W::SS, GS = W::GS, NT = W::NT, NWG = W::NWG;
-  extern __shared__ __attribute__((aligned(16))) float lds[];
-  float* stg = lds;                   // [2][DP][SS]
-  float* gm = lds + 2 * DP * SS;      // [DP][GS]
-  float* red = gm + DP * GS;          // [NWG]
+template <int TI, int NW>
+__global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW == 6 ? 3 : 2)))
+pe_wg_kernel(long long n, int d1, int d2, int ns, float eps, const void* X, void* Y, int dtype, int vec) {
+  using W = PEWg<TI, NW>;
+  using P = PESplit<W::DP, 32>;
+  using T32 = PESplit<32, 32>;
+  constexpr int NQ = W::NQ;
+  constexpr float XS = 4096.f, AS = 2048.f, BS = 4096.f;   // |X| <= 2, |G| <= 4, |B| <= 8 as fp16 operands
+  extern __shared__ __attribute__((aligned(16))) _Float16 wlds[];
+  const int w = __builtin_amdgcn_readfirstlane(wave_id()), lane = lane_id();
   const long long mat = blockIdx.x;
-  const int wv = wave_id(), lane = lane_id(), c = lane & 31, h = lane >> 5;
   const bool tall = d1 > d2;
   const int rows = tall ? d2 : d1, cols = tall ? d1 : d2;   // wide orientation
-  const int NJ = (cols + 31) / 32;                          // <= NWG
-  const bool own = wv < NJ;
-  const long long base = mat * (long long)d1 * d2;
-  f32x16 Xr[TI];
+  const int NJ = (cols + 31) / 32;                          // <= NW
+  const bool own = w < NJ;
+  float* red = reinterpret_cast<float*>(wlds + max(NJ * W::BLK, 2 * W::FR));
+  _Float16 *fG = wlds, *fB = wlds + W::FR;
+  const long long base = mat * (long long)d1 * d2 * (dtype == 0 ? 4 : 2);
+  const char* Xm = static_cast<const char*>(X) + base;
+  char* Ym = static_cast<char*>(Y) + base;
+
+  auto slot = [&](_Float16* m, int K, int I, int kb) { return m + ((K * TI + I) * 2 + kb) * 1024; };
+  auto put_frag = [&](_Float16* p, const SFrag& f) {
+    *reinterpret_cast<f16x8*>(p + lane * 8) = f.hi;
+    *reinterpret_cast<f16x8*>(p + 512 + lane * 8) = f.lo;
+  };
+  auto get_frag = [&](const _Float16* p) {
+    return SFrag{*reinterpret_cast<const f16x8*>(p + lane * 8), *reinterpret_cast<const f16x8*>(p + 512 + lane * 8)};
+  };
+  static_assert(T32::ELEMS == 2 * 1024, "a tile's transposing scratch is its slot");
+  auto share = [&](_Float16* m, const f32x16& t, int I, int I2, float s) {
 #pragma unroll
-  for (int I = 0; I < TI; ++I)
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int i = 32 * I + crow(r, h), j = 32 * wv + c;
-      float v = 0.f;
-      if (own && i < rows && j < cols) v = load_any(X, base + (tall ? (long long)j * d2 + i : (long long)i * d2 + j), dtype);
-      Xr[I][r] = v;
+    for (int kb = 0; kb < 2; ++kb) put_frag(slot(m, I, I2, kb), split_c(t, kb, s));
+    if (I != I2) {
+      const int l = opaque_lane();
+      _Float16* sc = slot(m, I2, I, 0);
+      T32::put_tile(t, s, sc, l);
+      const SFrag f0 = T32::get_tile(sc, 0, l), f1 = T32::get_tile(sc, 1, l);
+      put_frag(slot(m, I2, I, 0), f0);
+      put_frag(slot(m, I2, I, 1), f1);
     }
+  };
+
+  f32x16 Xr[TI];
+  auto each = [&](auto&& f) {   // f(I, r, offset or -1) over this lane's elements
+    const int l = opaque_lane(), c = l & 31, h = l >> 5, j = 32 * w + c;
+    const int si = tall ? 1 : cols, sj = tall ? rows : 1;
+#pragma unroll
+    for (int I = 0; I < TI; ++I)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int i = 32 * I + crow(r, h);
+        f(I, r, i < rows && j < cols ? i * si + j * sj : -1);
+      }
+  };
+  if (vec) {   // tall fp32, rows % 4 == 0, aligned: four consecutive rows of a column
+    const int c = lane & 31, h = lane >> 5, j = 32 * w + c;
+#pragma unroll
+    for (int I = 0; I < TI; ++I)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int i = 32 * I + 8 * q + 4 * h;
+        const bool ok = i < rows && j < cols;
+        const f32x4 v = *reinterpret_cast<const f32x4*>(reinterpret_cast<const float*>(Xm) + (ok ? j * rows + i : 0));
+#pragma unroll
+        for (int u = 0; u < 4; ++u) Xr[I][4 * q + u] = ok ? v[u] : 0.f;
+      }
+  } else if (dtype == 0) {
+    each([&](int I, int r, int o) { const float v = pe_ld1<0>(Xm, max(o, 0)); Xr[I][r] = o >= 0 ? v : 0.f; });
+  } else if (dtype == 1) {
+    each([&](int I, int r, int o) { const float v = pe_ld1<1>(Xm, max(o, 0)); Xr[I][r] = o >= 0 ? v : 0.f; });
+  } else {
+    each([&](int I, int r, int o) { const float v = pe_ld1<2>(Xm, max(o, 0)); Xr[I][r] = o >= 0 ? v : 0.f; });
+  }
   {
     float ss = 0.f;
 #pragma unroll
@@ -388,121 +451,113 @@ pe_wg_kernel(long long n, int d1, int d2, int ns, float eps, const void* X, void
 #pragma unroll
       for (int r = 0; r < 16; ++r) ss += Xr[I][r] * Xr[I][r];
     ss = wave_sum(ss);
-    if (lane == 0) red[wv] = ss;
+    if (lane == 0) red[w] = ss;
     __syncthreads();
     float tot = 0.f;
 #pragma unroll
-    for (int w = 0; w < NWG; ++w) tot += red[w];
+    for (int i = 0; i < NW; ++i) tot += red[i];
     const float inv = 1.f / (sqrtf(tot + eps) * 1.01f + 1e-6f);
 #pragma unroll
     for (int I = 0; I < TI; ++I) Xr[I] *= inv;
   }
   for (int st = 0; st < ns; ++st) {
     const float pa = kPE[st][0], pb = kPE[st][1], pc = kPE[st][2];
-    f32x16 G[NT];
+    if (own) {
+      f32x16 b[TI][1];
 #pragma unroll
-    for (int q = 0; q < NT; ++q) G[q] = zero16();
-    // ---- Gram over the staged column blocks
-    for (int J = 0; J < NJ; ++J) {
-      float* buf = stg + (J & 1) * DP * SS;
-      if (wv == J) {
-#pragma unroll
-        for (int I = 0; I < TI; ++I)
-#pragma unroll
-          for (int r = 0; r < 16; ++r) buf[(32 * I + crow(r, h)) * SS + c] = Xr[I][r];
-      }
-      __syncthreads();   // the block is staged; the reads of this buffer two blocks ago are done
-#pragma unroll
-      for (int q = 0; q < NT; ++q) {
-        const int t = wv + NWG * q;
-        if (t >= TI * TI) break;
-        const int I = t / TI, I2 = t % TI;
-        const float* ra = buf + (32 * I + c) * SS;
-        const float* rb = buf + (32 * I2 + c) * SS;
-#pragma unroll
-        for (int kb = 0; kb < 16; ++kb) G[q] = M::mma(M::ld_contig(ra, kb, h), M::ld_contig(rb, kb, h), G[q]);
-        __builtin_amdgcn_sched_barrier(0);
-      }
-    }
-    // ---- B = b G + c G^2
-#pragma unroll
-    for (int q = 0; q < NT; ++q) {
-      const int t = wv + NWG * q;
-      if (t >= TI * TI) break;
-      const int I = t / TI, I2 = t % TI;
-#pragma unroll
-      for (int r = 0; r < 16; ++r) gm[(32 * I + crow(r, h)) * GS + 32 * I2 + c] = G[q][r];
+      for (int I = 0; I < TI; ++I) b[I][0] = Xr[I];
+      P::put_block(b, 0, XS, wlds + w * W::BLK, opaque_lane());
     }
     __syncthreads();
-    f32x16 Bt[NT];
+    f32x16 G[NQ];
 #pragma unroll
-    for (int q = 0; q < NT; ++q) {
-      const int t = wv + NWG * q;
-      if (t >= TI * TI) break;
-      const int I = t / TI, I2 = t % TI;
-      f32x16 acc = zero16();
-#pragma unroll 1
+    for (int q = 0; q < NQ; ++q) {
+      G[q] = zero16();
+      if (w + NW * q < W::NT) {
+        int I, I2;
+        W::tile(w + NW * q, I, I2);
+        const int l = opaque_lane();
+#pragma unroll 2
+        for (int J = 0; J < NJ; ++J)
+#pragma unroll
+          for (int kb = 0; kb < 2; ++kb)
+            G[q] = mma_split(P::get(wlds + J * W::BLK, I, kb, l), P::get(wlds + J * W::BLK, I2, kb, l), G[q]);
+      }
+    }
+    __syncthreads();   // the staged blocks have been read
+#pragma unroll
+    for (int q = 0; q < NQ; ++q)
+      if (w + NW * q < W::NT) {
+        int I, I2;
+        W::tile(w + NW * q, I, I2);
+        G[q] *= 1.f / (XS * XS);
+        share(fG, G[q], I, I2, AS);
+      }
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < NQ; ++q)
+      if (w + NW * q < W::NT) {
+        int I, I2;
+        W::tile(w + NW * q, I, I2);
+        f32x16 a2 = zero16();
+#pragma unroll
+        for (int K = 0; K < TI; ++K)
+#pragma unroll
+          for (int kb = 0; kb < 2; ++kb)
+            a2 = mma_split(get_frag(slot(fG, K, I, kb)), get_frag(slot(fG, K, I2, kb)), a2);
+        share(fB, pb * G[q] + (pc / (AS * AS)) * a2, I, I2, BS);
+      }
+    __syncthreads();
+    if (own) {
+      f32x16 acc[TI];
+#pragma unroll
+      for (int I = 0; I < TI; ++I) acc[I] = zero16();
+#pragma unroll
       for (int K = 0; K < TI; ++K)
 #pragma unroll
-        for (int kb = 0; kb < 16; ++kb) {
-          // A: G[32I + m][32K + k]; B: G[32K + k][32I2 + n] (k = 2kb + h)
-          const float a = gm[(32 * I + c) * GS + 32 * K + 2 * kb + h];
-          const float b = gm[(32 * K + 2 * kb + h) * GS + 32 * I2 + c];
-          acc = M::mma(a, b, acc);
+        for (int kb = 0; kb < 2; ++kb) {
+          const SFrag x = split_c(Xr[K], kb, XS);
+#pragma unroll
+          for (int I = 0; I < TI; ++I) acc[I] = mma_split(get_frag(slot(fB, K, I, kb)), x, acc[I]);
+          __builtin_amdgcn_sched_barrier(0);   // keeps later fragments' loads from being hoisted (registers)
         }
-      Bt[q] = pb * G[q] + pc * acc;
-      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int I = 0; I < TI; ++I) Xr[I] = pa * Xr[I] + acc[I] * (1.f / (BS * XS));
     }
-    __syncthreads();   // every wave has read G
-#pragma unroll
-    for (int q = 0; q < NT; ++q) {
-      const int t = wv + NWG * q;
-      if (t >= TI * TI) break;
-      const int I = t / TI, I2 = t % TI;
-#pragma unroll
-      for (int r = 0; r < 16; ++r) gm[(32 * I + crow(r, h)) * GS + 32 * I2 + c] = Bt[q][r];
-    }
-    __syncthreads();
-    // ---- X <- a X + B X for this wave's column block (the next step's first
-    // barrier orders these reads of B before G overwrites it)
-    if (own) {
-      f32x16 Xn[TI];
-#pragma unroll
-      for (int I = 0; I < TI; ++I) {
-        Xn[I] = pa * Xr[I];
-#pragma unroll
-        for (int K = 0; K < TI; ++K) {
-#pragma unroll
-          for (int kb = 0; kb < 16; ++kb)
-            Xn[I] = M::mma(M::ld_cslot(gm + (32 * I + c) * GS + 32 * K, kb, h), M::from_c(Xr[K], kb), Xn[I]);
-          __builtin_amdgcn_sched_barrier(0);   // keeps the B loads of later blocks from being hoisted (registers)
-        }
-      }
-#pragma unroll
-      for (int I = 0; I < TI; ++I) Xr[I] = Xn[I];
-    }
+    __syncthreads();   // B has been read: the blocks may be staged over it
   }
   if (!own) return;
+  if (vec) {
+    const int l = opaque_lane(), c = l & 31, h = l >> 5, j = 32 * w + c;
 #pragma unroll
-  for (int I = 0; I < TI; ++I)
+    for (int I = 0; I < TI; ++I)
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int i = 32 * I + crow(r, h), j = 32 * wv + c;
-      if (i < rows && j < cols)
-        store_any(Y, base + (tall ? (long long)j * d2 + i : (long long)i * d2 + j), dtype, Xr[I][r]);
-    }
+      for (int q = 0; q < 4; ++q) {
+        const int i = 32 * I + 8 * q + 4 * h;
+        if (i < rows && j < cols)
+          *reinterpret_cast<f32x4*>(reinterpret_cast<float*>(Ym) + j * rows + i) =
+              f32x4{Xr[I][4 * q], Xr[I][4 * q + 1], Xr[I][4 * q + 2], Xr[I][4 * q + 3]};
+      }
+  } else if (dtype == 0) {
+    each([&](int I, int r, int o) { if (o >= 0) pe_st1<0>(Ym, o, Xr[I][r]); });
+  } else if (dtype == 1) {
+    each([&](int I, int r, int o) { if (o >= 0) pe_st1<1>(Ym, o, Xr[I][r]); });
+  } else {
+    each([&](int I, int r, int o) { if (o >= 0) pe_st1<2>(Ym, o, Xr[I][r]); });
+  }
 }
 
-template <int TI>
+template <int TI, int NW>
 atlas_status launch_wg(long long n, int d1, int d2, int ns, float eps, const void* X, void* Y, int dtype,
                        hipStream_t st) {
+  using W = PEWg<TI, NW>;
   if (n > 0x7fffffffLL) return fail(ATLAS_ERR_UNSUPPORTED_SHAPE, "n too large for the workgroup kernel");
-  static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(pe_wg_kernel<TI>),
-                                                     hipFuncAttributeMaxDynamicSharedMemorySize,
-                                                     (int)PEWg<TI>::lds_bytes());
+  static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(pe_wg_kernel<TI, NW>),
+                                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)W::lds_bytes(NW));
   if (attr != hipSuccess) return fail_hip(attr, "pe_wg attribute");
-  hipLaunchKernelGGL((pe_wg_kernel<TI>), dim3((unsigned)n), dim3(512), PEWg<TI>::lds_bytes(), st, n, d1, d2, ns, eps,
-                     X, Y, dtype);
+  const int vec = pe_path(d1, d2, 1, dtype, X, Y) == PE_TALL4, nj = (std::max(d1, d2) + 31) / 32;
+  hipLaunchKernelGGL((pe_wg_kernel<TI, NW>), dim3((unsigned)n), dim3(64 * NW), W::lds_bytes(nj), st, n, d1, d2, ns, eps,
+                     X, Y, dtype, vec);
   const hipError_t e = hipGetLastError();
   return e == hipSuccess ? ATLAS_OK : fail_hip(e, "pe_batched launch");
 }
@@ -557,8 +612,10 @@ template <class M>
 atlas_status dispatch(long long n, int d1, int d2, int ns, float eps, const void* X, void* Y, int dtype,
                       hipStream_t st) {
   const int rows = d1 < d2 ? d1 : d2, cols = d1 < d2 ? d2 : d1;
-  if (rows > 64) return rows <= 96 ? launch_wg<3>(n, d1, d2, ns, eps, X, Y, dtype, st)
-                                   : launch_wg<4>(n, d1, d2, ns, eps, X, Y, dtype, st);
+  // six waves (two workgroups on a CU) where the columns fit them
+  if (rows > 96) return launch_wg<4, 8>(n, d1, d2, ns, eps, X, Y, dtype, st);
+  if (rows > 64) return cols <= 192 ? launch_wg<3, 6>(n, d1, d2, ns, eps, X, Y, dtype, st)
+                                    : launch_wg<3, 8>(n, d1, d2, ns, eps, X, Y, dtype, st);
   const int D = rows <= 32 ? 32 : 64;
   if (cols > 128) return D == 32 ? launch_pair<M, 32>(n, d1, d2, ns, eps, X, Y, dtype, st)
                                  : launch_pair<M, 64>(n, d1, d2, ns, eps, X, Y, dtype, st);

@@ -101,12 +101,14 @@ struct PESplit {
   static constexpr int TI = D / 32, TJ = E / 32;
   static constexpr int BLOCK = 32 * D;
   static constexpr int ELEMS = 2 * BLOCK;
-  static_assert(D == 32 || D == 64, "units per row");
+  static_assert(D == 32 || D == 64 || D == 96 || D == 128, "units per row");
 
-  // 8-byte unit u of row r: D 64 (two rows span the banks) u ^ g, g's top bit
-  // that of r / 2 modulo 2, the other three r / 4; D 32 (four rows) u ^ (r / 4).
+  // 8-byte unit u of row r lies at u ^ g(r).  The low three bits of g are r / 4
+  // (eight different units of a write to rows that share their banks); where
+  // the four rows of a transposing read share banks too (two rows span them at
+  // D 64, one at D 128), the bits above separate those.
   __device__ __forceinline__ static int at(int r, int u) {
-    const int g = D == 64 ? ((r >> 1 & 1) << 3) | (r >> 2 & 7) : (r >> 2 & 7);
+    const int g = (r >> 2 & 7) | (D == 64 ? (r >> 1 & 1) << 3 : D == 128 ? (r & 3) << 3 : 0);
     return r * D + 4 * (u ^ g);
   }
   __device__ __forceinline__ static void put4(const f32x16& t, int q, float s, _Float16* p) {
