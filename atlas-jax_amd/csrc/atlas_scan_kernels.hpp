@@ -363,6 +363,8 @@ prep_kernel(ScanArgs p) {
 // Row t of the chunk is owned by thread t (cs <= CS_MAX; the block holds cs
 // rounded up to whole waves).  The two cs x (cs+1) tables are sized by the
 // runtime cs (coef_lds_bytes(cs)), so at cs = 64 four blocks share a CU.
+// Bound by one wave's chain of LDS reads: cs = 64, 64 blocks, 19 us (33 us with
+// per-thread ranges, which wait for every read, and a division per element).
 //   c[t,i] = (2/D) g'_i sum_{s=i}^{min(t,i+w-1)} theta(s->t) (-eta_s),
 //   evaluated as g'_i (R_t[i] - R_t[i+w]) with suffix sums
 //   R_t[s] = sum_{u=s}^{t} theta(u->t) (-eta_u).
@@ -387,81 +389,129 @@ coef_kernel(ScanArgs p, int c0, int nwin) {
   }
   __syncthreads();
   const long long tb = chunk_table(p, stream, chunk);
-  if (t < cs) {
+  // Every loop below runs over the same tokens in every thread (a thread's own
+  // range is a predicate) in steps of four (cs is a multiple of 4), whose reads
+  // are all issued before their first use.
+  const bool row = t < cs;
+  float* Rt = R + (row ? t : 0) * CP;
+  float* Ct = C + (row ? t : 0) * CP;
+  {
     float th = 1.f, apv = 1.f;
-    for (int r = 0; r <= t; ++r) { th *= gt[r]; apv *= ga[r]; }
-    p.thp[tb * cs + t] = th;
-    p.ap[tb * cs + t] = apv;
-    // Window sums sum_{s=i}^{min(t, i+w-1)} m_t[s], m_t[s] = theta(s->t)
-    // (-eta_s) (0 past t), without subtraction: over blocks of w tokens, the
-    // in-block suffix sums (into Rt) and prefix sums (into Ct); a window is
-    // the suffix of its first block plus, when it is not block-aligned, the
-    // prefix of the next block.  (The difference of two suffix sums
-    // R_t[i] - R_t[i+w] cancels for windows far behind t, where the decayed
-    // window is much smaller than the sums.)  All terms share the sign of
-    // -eta.  One backward pass forms m_t (kept in Ct) and the suffix sums,
-    // one forward pass turns Ct into the prefix sums in place.
-    const int w = p.w_eff;
-    float* __restrict__ Rt = R + t * CP;
-    float* __restrict__ Ct = C + t * CP;
-    for (int s = cs - 1; s > t; --s) {
-      Rt[s] = 0.f;
-      Ct[s] = 0.f;
+    for (int r0 = 0; r0 < cs; r0 += 4) {
+      float g1[4], g2[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) { g1[u] = gt[r0 + u]; g2[u] = ga[r0 + u]; }
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        th = r0 + u <= t ? th * g1[u] : th;
+        apv = r0 + u <= t ? apv * g2[u] : apv;
+      }
     }
+    if (row) {
+      p.thp[tb * cs + t] = th;
+      p.ap[tb * cs + t] = apv;
+    }
+  }
+  // Window sums sum_{s=i}^{min(t, i+w-1)} m_t[s], m_t[s] = theta(s->t)
+  // (-eta_s) (0 past t), without subtraction: over blocks of w tokens, the
+  // in-block suffix sums (into Rt) and prefix sums (into Ct); a window is
+  // the suffix of its first block plus, when it is not block-aligned, the
+  // prefix of the next block.  (The difference of two suffix sums
+  // R_t[i] - R_t[i+w] cancels for windows far behind t, where the decayed
+  // window is much smaller than the sums.)  All terms share the sign of
+  // -eta.  One backward pass forms m_t (kept in Ct) and the suffix sums,
+  // one forward pass turns Ct into the prefix sums in place.
+  const int w = p.w_eff;
+  float m = 0.f;
+  if (row) {
     {
       float prod = 1.f, suf = 0.f;
-#pragma unroll 8
-      for (int s = t, r = t % w; s >= 0; --s) {
-        const float mv = prod * (-ge[s]);
-        prod *= gt[s];
-        suf = (r == w - 1 || s == t) ? mv : suf + mv;
-        Rt[s] = suf;
-        Ct[s] = mv;
-        r = (r == 0) ? w - 1 : r - 1;
+      int r = (cs - 1) % w;
+      for (int s0 = cs - 4; s0 >= 0; s0 -= 4) {
+        float e1[4], g1[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) { e1[u] = ge[s0 + u]; g1[u] = gt[s0 + u]; }
+#pragma unroll
+        for (int u = 3; u >= 0; --u) {
+          const int s = s0 + u;
+          const float mv = prod * (-e1[u]);
+          prod = s <= t ? prod * g1[u] : prod;
+          suf = (r == w - 1 || s == t) ? mv : suf + mv;
+          Rt[s] = s <= t ? suf : 0.f;
+          Ct[s] = s <= t ? mv : 0.f;
+          r = (r == 0) ? w - 1 : r - 1;
+        }
       }
       float pre = 0.f;
-#pragma unroll 8
-      for (int s = 0, r = 0; s < cs; ++s) {   // (past t the block's prefix stays its sum up to t)
-        pre = (r == 0) ? Ct[s] : pre + Ct[s];
-        Ct[s] = pre;
-        if (++r == w) r = 0;
+      r = 0;
+      for (int s0 = 0; s0 < cs; s0 += 4) {   // (past t the block's prefix stays its sum up to t)
+        float c1[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) c1[u] = Ct[s0 + u];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          pre = (r == 0) ? c1[u] : pre + c1[u];
+          Ct[s0 + u] = pre;
+          if (++r == w) r = 0;
+        }
       }
     }
     const float scale = 2.f / (float)p.D;
-    float m = 0.f;
-#pragma unroll 8
-    for (int i = 0; i < cs; ++i) {
-      float cv = 0.f;
-      if (i <= t) {
-        const int jw = min(i + w - 1, cs - 1);
-        float win = Rt[i];
-        if (jw / w != i / w) win += Ct[jw];
-        cv = scale * gg[i] * win;
+    int jn = w;   // the first token of the block after i's
+    for (int i0 = 0; i0 < cs; i0 += 4) {
+      float win[4], nextp[4], g1[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        win[u] = Rt[i0 + u];
+        nextp[u] = Ct[min(i0 + u + w - 1, cs - 1)];
+        g1[u] = gg[i0 + u];
       }
-      Ct[i] = cv;   // the prefix sum at i was last read for window i - w + 1 <= i
-      m = fmaxf(m, fabsf(cv));
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int i = i0 + u;
+        if (i == jn) jn += w;
+        const float wv = min(i + w - 1, cs - 1) >= jn ? win[u] + nextp[u] : win[u];
+        const float cv = i <= t ? scale * g1[u] * wv : 0.f;
+        Rt[i] = cv;
+        m = fmaxf(m, fabsf(cv));
+      }
     }
-    mr[t] = (m > 0.f) ? m : 1.f;
-    p.cm[tb * cs + t] = mr[t];
-  }
-  __syncthreads();
-  // a(s->t) row t into R (R is no longer needed)
-  if (t < cs) {
+    m = (m > 0.f) ? m : 1.f;
+    mr[t] = m;
+    p.cm[tb * cs + t] = m;
+    // a(s->t) row t into Ct (the prefix sums are no longer needed)
     float prod = 1.f;
-    for (int s = cs - 1; s > t; --s) R[t * CP + s] = 0.f;
-    R[t * CP + t] = 1.f;
-    for (int s = t - 1; s >= 0; --s) {
-      prod *= ga[s + 1];
-      R[t * CP + s] = prod;
+    for (int s0 = cs - 4; s0 >= 0; s0 -= 4) {
+      float g1[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) g1[u] = ga[min(s0 + u + 1, cs - 1)];
+#pragma unroll
+      for (int u = 3; u >= 0; --u) {
+        const int s = s0 + u;
+        prod = s < t ? prod * g1[u] : 1.f;
+        Ct[s] = s <= t ? prod : 0.f;
+      }
     }
   }
   __syncthreads();
+  // column t of every row
   float* cmt = p.cmt + tb * cs * cs;
   float* am = p.am + tb * cs * cs;
-  for (int idx = t; idx < cs * cs; idx += blockDim.x) {
-    const int r = idx / cs, i = idx % cs;
-    cmt[idx] = C[r * CP + i] / mr[r];
-    am[idx] = R[r * CP + i];
+  if (row) {
+    for (int r0 = 0; r0 < cs; r0 += 4) {
+      float c1[4], m1[4], a1[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        c1[u] = R[(r0 + u) * CP + t];
+        m1[u] = mr[r0 + u];
+        a1[u] = C[(r0 + u) * CP + t];
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        cmt[(r0 + u) * cs + t] = c1[u] / m1[u];
+        am[(r0 + u) * cs + t] = a1[u];
+      }
+    }
   }
 }
 
