@@ -336,9 +336,10 @@ def _layer_prologue_bwd_supported(meta):
     return D in (16, 32, 64) and 1 <= K <= 4 and H * D <= 1024 and n_gates * H <= threads
 
 
-def _layer_prologue_bwd_hip(proj, cw, cb, pc, gb, meta, gq, gk, gv, ggates, gr):
-    """atlas_layer_prologue_bwd: (d proj, d conv_w, d conv_b, d poly, d gate_b)
-    for the cotangents of (q, k, v, gates, retrieve) (None = zero)."""
+def _layer_prologue_bwd_hip(proj, cw, cb, pc, gb, meta, gq, gk, gv, ggates, gr, dproj_dtype=torch.float32):
+    """atlas_layer_prologue_bwd_as: (d proj, d conv_w, d conv_b, d poly, d gate_b)
+    for the cotangents of (q, k, v, gates, retrieve) (None = zero); all fp32, or
+    d proj in dproj_dtype (the same values rounded as they are stored)."""
     B, T, H, D, K, poly_degree, n_gates, has_r, max_lr, dtype = meta
     dev = proj.device
     proj = proj.contiguous()
@@ -353,7 +354,9 @@ def _layer_prologue_bwd_hip(proj, cw, cb, pc, gb, meta, gq, gk, gv, ggates, gr):
     ggates = ct(ggates, (n_gates, B, T, H), torch.float32)
     gr = ct(gr, (B, T, H), torch.float32) if has_r else None
     ld = proj.shape[1]
-    dproj = torch.zeros(proj.shape, dtype=torch.float32, device=dev)
+    # (every one of the projection's columns is written)
+    exact = ld == 3 * H * D + (n_gates + int(has_r)) * H
+    dproj = (torch.empty if exact else torch.zeros)(proj.shape, dtype=dproj_dtype, device=dev)
     dcw = torch.empty_like(cwf)
     dcb = torch.empty_like(cbf)
     dgb = torch.empty_like(gbf)
@@ -361,11 +364,12 @@ def _layer_prologue_bwd_hip(proj, cw, cb, pc, gb, meta, gq, gk, gv, ggates, gr):
     lib = L.get_lib()
     ws_bytes = lib.atlas_layer_prologue_bwd_workspace_size(B, T, H, D, K, poly_degree, n_gates)
     ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
-    L.check(lib.atlas_layer_prologue_bwd(B, T, H, D, K, poly_degree, n_gates, int(has_r), L.ptr(proj), ld,
-                                         L.dtype_code(proj.dtype), L.ptr(cwf), L.ptr(cbf), L.ptr(pcf), L.ptr(gbf),
-                                         max_lr, L.ptr(gq), L.ptr(gk), L.ptr(gv), L.dtype_code(gdt), L.ptr(ggates),
-                                         L.ptr(gr), L.ptr(dproj), ld, L.ptr(dcw), L.ptr(dcb), L.ptr(dpc),
-                                         L.ptr(dgb), L.ptr(ws), ws_bytes, L.stream_ptr(dev)))
+    L.check(lib.atlas_layer_prologue_bwd_as(B, T, H, D, K, poly_degree, n_gates, int(has_r), L.ptr(proj), ld,
+                                            L.dtype_code(proj.dtype), L.ptr(cwf), L.ptr(cbf), L.ptr(pcf), L.ptr(gbf),
+                                            max_lr, L.ptr(gq), L.ptr(gk), L.ptr(gv), L.dtype_code(gdt), L.ptr(ggates),
+                                            L.ptr(gr), L.ptr(dproj), ld, L.dtype_code(dproj_dtype), L.ptr(dcw),
+                                            L.ptr(dcb), L.ptr(dpc), L.ptr(dgb), L.ptr(ws), ws_bytes,
+                                            L.stream_ptr(dev)))
     return dproj, dcw, dcb, dpc, dgb
 
 
@@ -433,8 +437,8 @@ class LayerPrologue(torch.autograd.Function):
         pc = pc if ctx.has_pc else None
         if _layer_prologue_bwd_supported(ctx.meta):
             dproj, dcw, dcb, dpc, dgb = _layer_prologue_bwd_hip(proj, cw, cb, pc, gb, ctx.meta, gq, gk, gv, ggates,
-                                                                gr if ctx.meta[7] else None)
-            return (dproj.to(proj.dtype), dcw.to(cw.dtype), dcb.to(cb.dtype),
+                                                                gr if ctx.meta[7] else None, proj.dtype)
+            return (dproj, dcw.to(cw.dtype), dcb.to(cb.dtype),
                     None if pc is None else dpc.to(pc.dtype), dgb.to(gb.dtype), None)
         ins = [t.detach().requires_grad_(True) if t is not None else None for t in (proj, cw, cb, pc, gb)]
         with torch.enable_grad():

@@ -261,3 +261,40 @@ def test_layer_prologue_backward(dtype, poly, H, D, K, n_gates, has_r, T):
     grads = torch.autograd.grad([o for o, _ in pairs], [t for t in leaves_d if t is not None], [c for _, c in pairs])
     for a, b_ in zip(grads, gl):
         assert torch.equal(a, b_.to(a.dtype))
+
+
+@pytest.mark.parametrize("dtype,H,D,K,ld_extra,T", [("bf16", 8, 64, 4, 0, 63), ("f16", 12, 64, 4, 0, 129),
+                                                    ("f32", 4, 32, 4, 0, 5), ("bf16", 8, 64, 4, 1, 66),
+                                                    ("bf16", 5, 16, 4, 0, 64), ("f32", 16, 64, 3, 0, 70)])
+def test_layer_prologue_paths(dtype, H, D, K, ld_extra, T):
+    """The prologue's forward and backward on every load path (rows aligned to
+    four elements in each dtype, a row stride that is not, conv kernels below
+    4, one to eight groups of threads, runs that end mid-block) against the
+    same arithmetic in torch (layer_prologue_reference_ops, fp32) and its
+    autograd: the 16-bit outputs within one rounding (2^-8 bf16, 2^-11 fp16),
+    fp32 sums of up to 2 T terms within 1e-5."""
+    torch = _torch()
+    from atlas_amd.memory_layer import (_layer_prologue_bwd_hip, _layer_prologue_hip, layer_prologue_reference_ops)
+    tdt = {"f32": torch.float32, "bf16": torch.bfloat16, "f16": torch.float16}[dtype]
+    B, HD = 2, H * D
+    g = torch.Generator(device="cuda").manual_seed(H * D + T)
+    wide = torch.randn(B * T, 3 * HD + 5 * H + ld_extra, device="cuda", generator=g).to(tdt)
+    cw = torch.randn(3, HD, K, device="cuda", generator=g) * 0.5
+    cb = torch.randn(3, HD, device="cuda", generator=g) * 0.1
+    pc = torch.tensor([1.0, 0.5], device="cuda")
+    gb = torch.randn(4, H, device="cuda", generator=g)
+    meta = (B, T, H, D, K, 2, 4, True, 0.1, tdt)
+    ins = [t.float().requires_grad_(True) for t in (wide, cw, cb, pc, gb)]
+    ref = layer_prologue_reference_ops(*ins, meta[:-1] + (torch.float32,))
+    got = _layer_prologue_hip(wide, cw, cb, pc, gb, meta)
+    one = {"f32": 1e-5, "bf16": 2.0 ** -8, "f16": 2.0 ** -11}[dtype]
+    rel = lambda a, b: float((a.double() - b.double()).norm() / b.double().norm())  # noqa: E731
+    for i, (a, b) in enumerate(zip(got, ref)):
+        assert rel(a, b) <= (one if i < 3 else 1e-5), i
+    cts = [torch.randn(B, T, H, D, device="cuda", generator=g).to(tdt) for _ in range(3)] + \
+        [torch.randn(4, B, T, H, device="cuda", generator=g), torch.randn(B, T, H, device="cuda", generator=g)]
+    want = torch.autograd.grad(ref, ins, [c.float() for c in cts])
+    for dt in {torch.float32, tdt}:
+        grads = _layer_prologue_bwd_hip(wide, cw, cb, pc, gb, meta, *cts, dproj_dtype=dt)
+        for i, (a, b) in enumerate(zip(grads, want)):
+            assert a.shape == b.shape and rel(a, b) <= (1e-5 if i or dt == torch.float32 else one), (i, dt)
