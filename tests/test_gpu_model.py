@@ -288,7 +288,7 @@ def test_layer_prologue_paths(dtype, H, D, K, ld_extra, T):
     ref = layer_prologue_reference_ops(*ins, meta[:-1] + (torch.float32,))
     got = _layer_prologue_hip(wide, cw, cb, pc, gb, meta)
     one = {"f32": 1e-5, "bf16": 2.0 ** -8, "f16": 2.0 ** -11}[dtype]
-    rel = lambda a, b: float((a.double() - b.double()).norm() / b.double().norm())  # noqa: E731
+    rel = lambda a, b: float((a.detach().double() - b.detach().double()).norm() / b.detach().double().norm())  # noqa
     for i, (a, b) in enumerate(zip(got, ref)):
         assert rel(a, b) <= (one if i < 3 else 1e-5), i
     cts = [torch.randn(B, T, H, D, device="cuda", generator=g).to(tdt) for _ in range(3)] + \
