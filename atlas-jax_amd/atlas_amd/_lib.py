@@ -59,6 +59,8 @@ def _declare(lib):
     lib.atlas_scan_workspace_size.argtypes = [ctypes.POINTER(ScanDesc)]
     lib.atlas_scan_fwd.restype = ctypes.c_int
     lib.atlas_scan_fwd.argtypes = [ctypes.POINTER(ScanDesc)] + [_P] * 7 + [_P] * 4 + [_P, _P, sz, _P]
+    lib.atlas_scan_fwd_from.restype = ctypes.c_int
+    lib.atlas_scan_fwd_from.argtypes = [ctypes.POINTER(ScanDesc)] + [_P] * 7 + [_P] * 8 + [_P, _P, _P, sz, _P]
     lib.atlas_scan_noalloc_scratch_bytes.restype = sz
     lib.atlas_scan_noalloc_scratch_bytes.argtypes = []
     lib.atlas_scan_fwd_noalloc.restype = ctypes.c_int

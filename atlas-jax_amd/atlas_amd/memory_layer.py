@@ -221,8 +221,8 @@ def memory_scan(q, k, v, alpha, eta, theta, gamma, state, chunk_size, omega_wind
 
 def _scan_forward(q, k, v, alpha, eta, theta, gamma, state, chunk_size, omega_window, ns_steps, precision=None,
                   n_slices=0, trace=False):
-    """memory_scan's forward on the library (no autograd).  With trace=True
-    (atlas_scan_fwd_trace) also returns the chunk-start states, a
+    """memory_scan's forward on the library (no autograd, out of place:
+    atlas_scan_fwd_from).  With trace=True also returns the chunk-start states, a
     (n_chunks, 4, B, H, D*E) fp32 tensor (W1, W2, S1, S2 per chunk)."""
     B, T, H, D = q.shape
     E = state.W1.shape[-1]
@@ -234,9 +234,12 @@ def _scan_forward(q, k, v, alpha, eta, theta, gamma, state, chunk_size, omega_wi
     for name, t in (("alpha", al), ("eta", et), ("theta", th)):
         if tuple(t.shape) != (B, T, H):
             raise ValueError(f"{name} shape {tuple(t.shape)} != {(B, T, H)}")
-    W1, W2, S1, S2 = (t.float().contiguous().clone() for t in state)
-    if tuple(W1.shape) != (B, H, D, E) or tuple(W2.shape) != (B, H, E, D):
+    st = [t.float().contiguous() for t in state]
+    if tuple(st[0].shape) != (B, H, D, E) or tuple(st[1].shape) != (B, H, E, D):
         raise ValueError("state shapes do not match (B, H, D, E) / (B, H, E, D)")
+    # the scan reads the state in 16-byte rows (a view may start anywhere)
+    st = [t if t.data_ptr() % 16 == 0 else t.clone() for t in st]
+    out = [torch.empty_like(t) for t in st]
     y = torch.empty_like(qc)
     desc = L.ScanDesc(B=B, T=T, H=H, D=D, E=E, chunk_size=chunk_size, omega_window=omega_window,
                       ns_steps=ns_steps, io_dtype=L.dtype_code(io), gate_dtype=L.dtype_code(gdt),
@@ -246,15 +249,10 @@ def _scan_forward(q, k, v, alpha, eta, theta, gamma, state, chunk_size, omega_wi
     if ws_bytes == 0:
         raise L.AtlasError(1, lib.atlas_last_error().decode(errors="replace"))
     ws = torch.empty(ws_bytes, dtype=torch.uint8, device=q.device)
-    args = (L.ptr(qc), L.ptr(kc), L.ptr(vc), L.ptr(al), L.ptr(et), L.ptr(th), L.ptr(ga), L.ptr(W1), L.ptr(W2),
-            L.ptr(S1), L.ptr(S2), L.ptr(y))
-    if not trace:
-        L.check(lib.atlas_scan_fwd(desc, *args, L.ptr(ws), ws_bytes, L.stream_ptr(q.device)))
-        return y, DeepMemoryState(W1, W2, S1, S2)
-    n_chunks = -(-T // chunk_size)
-    tr = torch.empty(n_chunks, 4, B, H, D * E, dtype=torch.float32, device=q.device)
-    L.check(lib.atlas_scan_fwd_trace(desc, *args, L.ptr(tr), L.ptr(ws), ws_bytes, L.stream_ptr(q.device)))
-    return y, DeepMemoryState(W1, W2, S1, S2), tr
+    tr = torch.empty(-(-T // chunk_size), 4, B, H, D * E, dtype=torch.float32, device=q.device) if trace else None
+    L.check(lib.atlas_scan_fwd_from(desc, *(L.ptr(t) for t in (qc, kc, vc, al, et, th, ga, *st, *out, y, tr, ws)),
+                                    ws_bytes, L.stream_ptr(q.device)))
+    return (y, DeepMemoryState(*out), tr) if trace else (y, DeepMemoryState(*out))
 
 
 # ---------------------------------------------------------------------------

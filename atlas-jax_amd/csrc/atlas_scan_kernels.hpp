@@ -44,7 +44,7 @@ struct ScanArgs {
   long long xsb, xst, xsh, gsb, gst;
   const void *q, *k, *v, *alpha, *eta, *theta, *gamma;
   void* y;
-  float* W1[2];
+  float* W1[2];   // [cur]: the chunk's start state, [cur ^ 1]: its end state
   float* W2[2];
   float* S1[2];
   float* S2[2];

@@ -126,6 +126,22 @@ atlas_status atlas_scan_fwd(const atlas_scan_desc* desc,
                             void* y, void* workspace, size_t workspace_bytes,
                             void* stream);
 
+/* atlas_scan_fwd out of place: starts from W1_init .. S2_init (only read) and
+ * writes the final state to W1 .. S2, without the copies that an in-place
+ * call needs to keep its initial state.  The initial arrays may overlap none
+ * of the outputs.  state_trace: as in atlas_scan_fwd_trace, or NULL.  Same
+ * shapes, workspace and errors as atlas_scan_fwd. */
+atlas_status atlas_scan_fwd_from(const atlas_scan_desc* desc,
+                                 const void* q, const void* k, const void* v,
+                                 const void* alpha, const void* eta,
+                                 const void* theta, const void* gamma,
+                                 const float* W1_init, const float* W2_init,
+                                 const float* S1_init, const float* S2_init,
+                                 float* W1, float* W2, float* S1, float* S2,
+                                 void* y, float* state_trace,
+                                 void* workspace, size_t workspace_bytes,
+                                 void* stream);
+
 /* atlas_scan_fwd without a caller-provided workspace, for callers that
  * cannot allocate device memory (code under HIP graph capture, tight serving
  * loops, harnesses that forbid hipMalloc).  No counterpart in the reference.

@@ -303,3 +303,40 @@ def test_c3_benchmark_launch_192_streams():
     waves kernels, 4 slices, 768 workgroups in three rounds."""
     sample = [(0, 0), (5, 11), (10, 4), (15, 11)]
     _launch_case(16, 12, 64, 256, 64, 64, 5, "rand", seed=62, sample=sample)
+
+
+@pytest.mark.parametrize("n_chunks", [1, 2, 3])
+@pytest.mark.parametrize("D,E,cs,compute", [(64, 128, 64, "f16"), (64, 64, 128, "f16"), (32, 64, 64, "f32"),
+                                            (64, 256, 64, "f16"), (48, 64, 16, "f32")])
+def test_scan_from_equals_in_place(D, E, cs, compute, n_chunks):
+    """atlas_scan_fwd_from on every driver (tails with and without the slice
+    prefixes, fp32, wide, per-token) and chunk-count parity: the same y, final
+    state and chunk-start states, bit for bit, as atlas_scan_fwd_trace in
+    place on a copy, and the initial state untouched."""
+    import torch
+    from atlas_amd import _lib as L
+    B, H, T = 2, 3, n_chunks * cs - 1
+    g = torch.Generator(device="cuda").manual_seed(D + E + n_chunks)
+    rnd = lambda *s: torch.randn(*s, device="cuda", generator=g)  # noqa: E731
+    x = [rnd(B, T, H, D) * 0.3 for _ in range(3)]
+    gates = [torch.sigmoid(rnd(B, T, H)) for _ in range(4)]
+    init = [rnd(B, H, D, E) * 0.05, rnd(B, H, E, D) * 0.05, rnd(B, H, D, E) * 0.05, rnd(B, H, E, D) * 0.05]
+    desc = L.ScanDesc(B=B, T=T, H=H, D=D, E=E, chunk_size=cs, omega_window=8, ns_steps=5, io_dtype=0, gate_dtype=0,
+                      compute=L.COMPUTE_F16 if compute == "f16" else L.COMPUTE_F32)
+    lib = L.get_lib()
+    nb = lib.atlas_scan_workspace_size(desc)
+    ws = torch.empty(nb, dtype=torch.uint8, device="cuda")
+    run = {}
+    for how in ("from", "place"):
+        st0, y = [t.clone() for t in init], torch.empty_like(x[0])
+        tr = torch.empty(n_chunks, 4, B * H * D * E, device="cuda")
+        out = [torch.empty_like(t) for t in st0] if how == "from" else st0
+        ptrs = [L.ptr(t) for t in (*x, *gates, *(st0 if how == "from" else ()), *out, y, tr, ws)]
+        fn = lib.atlas_scan_fwd_from if how == "from" else lib.atlas_scan_fwd_trace
+        L.check(fn(desc, *ptrs, nb, L.stream_ptr(x[0].device)))
+        run[how] = [*out, y, tr]
+        if how == "from":
+            assert all(torch.equal(a, b) for a, b in zip(st0, init))
+            bad = [L.ptr(t) for t in (*x, *gates, *st0, st0[0], *out[1:], y, tr, ws)]
+            assert lib.atlas_scan_fwd_from(desc, *bad, nb, L.stream_ptr(x[0].device)) == 1   # overlapping states
+    assert all(torch.equal(a, b) for a, b in zip(run["from"], run["place"]))
