@@ -669,8 +669,8 @@ extern "C" atlas_status atlas_scan_fwd_trace(const atlas_scan_desc* d, const voi
 
 // One call of one chunk needs no copy of the state at all, where a caller that
 // keeps its initial state needed four clones before the in-place scan and four
-// copies after an odd chunk count: B1 T256 H16 335 -> 332 us, B8 T192 fp32
-// 386 -> 380, B8 T256 H8 586 -> 577, an 8-layer model on 60 tokens 2.98 -> 2.80 ms
+// copies after an odd chunk count: B1 T256 H16 335 -> 332 us, fp32 B1 T512 H4
+// D32 E32 386 -> 380, B8 T256 H8 586 -> 577, an 8-layer model on 60 tokens 2.98 -> 2.80 ms
 // (host bound: 64 launches fewer).
 extern "C" atlas_status atlas_scan_fwd_from(const atlas_scan_desc* d, const void* q, const void* k, const void* v,
                                             const void* alpha, const void* eta, const void* theta,

@@ -1760,8 +1760,11 @@ atlas_status pe_vjp_both(long long n, int D, int E, int ns, const float* X0, flo
 }
 
 size_t vjp_scratch_floats(int D, int E, int ns) {
-  // the fp32 VJP's per-workgroup scratch (the fp16 VJP needs none)
-  return (size_t)VJP_GRID * (ns > 1 ? ns - 1 : 1) * D * E;
+  // the fp32 VJP's per-workgroup scratch (the fp16 VJP needs none).  Callers
+  // keep workspaces by the size this reports: at 64 x 256 it stays what it was
+  // when two further 64 x 257 arrays lay in it.
+  const size_t extra = D == 64 && E == 256 ? (size_t)2 * 64 * 257 : 0;
+  return (size_t)VJP_GRID * ((size_t)(ns > 1 ? ns - 1 : 1) * D * E + extra);
 }
 
 // Shapes the backward is compiled for.
