@@ -77,6 +77,8 @@ def _declare(lib):
     lib.atlas_profile_read.argtypes = [i32, ctypes.POINTER(ctypes.c_int64), ctypes.POINTER(ctypes.c_double)]
     lib.atlas_profile_mfma_rate.restype = ctypes.c_int
     lib.atlas_profile_mfma_rate.argtypes = [i32, ctypes.POINTER(ctypes.c_double), _P]
+    lib.atlas_rms_norm.restype = ctypes.c_int
+    lib.atlas_rms_norm.argtypes = [i64, i32, _P, _P, i32, _P]
     lib.atlas_layer_prologue.restype = ctypes.c_int
     lib.atlas_layer_prologue.argtypes = ([i32] * 8 + [_P, i64, i32] + [_P] * 4 + [ctypes.c_float] +
                                          [_P] * 3 + [i32] + [_P, _P, _P])

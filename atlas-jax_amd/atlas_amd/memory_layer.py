@@ -259,8 +259,30 @@ def _scan_forward(q, k, v, alpha, eta, theta, gamma, state, chunk_size, omega_wi
 # Dense prologue helpers (torch) and the layer
 # ---------------------------------------------------------------------------
 
+_RMS_DTYPES = (torch.float32, torch.bfloat16, torch.float16)
+
+
+def _transformed(x):
+    """Whether a call on x is seen by more than eager autograd: functorch
+    wrappers, an open forward-mode level, graph tracing, dispatch modes."""
+    return (torch._C._functorch.is_functorch_wrapped_tensor(x) or torch.autograd.forward_ad._current_level >= 0
+            or torch.jit.is_tracing() or torch.compiler.is_compiling()
+            or torch._C._len_torch_dispatch_stack() > 0)
+
+
 def rms_norm(x):
-    """memory_layer.py:211-216: computed in fp32, returned in x's dtype."""
+    """memory_layer.py:211-216: computed in fp32, returned in x's dtype.
+    Plain dense GPU tensors with nothing to differentiate take one kernel;
+    everything else (gradients, forward-mode and vmap wrappers, tracing,
+    subclasses, CPU, other dtypes and layouts) the torch operations."""
+    if (type(x) in (torch.Tensor, nn.Parameter) and x.is_cuda and x.dtype in _RMS_DTYPES and x.dim() > 0
+            and x.numel() > 0 and x.is_contiguous() and not (x.requires_grad and torch.is_grad_enabled())
+            and x.device.index == torch.cuda.current_device() and not _transformed(x)):
+        y = torch.empty_like(x)
+        C = x.shape[-1]
+        L.check(L.get_lib().atlas_rms_norm(x.numel() // C, C, L.ptr(x), L.ptr(y), L.dtype_code(x.dtype),
+                                           L.stream_ptr(x.device)))
+        return y
     xf = x.float()
     return (xf * torch.rsqrt(xf.pow(2).mean(-1, keepdim=True) + 1e-6)).to(x.dtype)
 

@@ -13,6 +13,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <type_traits>
 
 #include "atlas_common.hpp"
 #include "atlas_scan.h"
@@ -23,6 +24,7 @@ namespace {
 
 constexpr int PRO_WAVES = 4;   // token-heads per workgroup
 constexpr int PRO_CH = 2;      // channels per lane (head dims up to 2 x 64)
+constexpr int RMS_WAVES = 4;   // rows per workgroup of the row norm
 
 struct ProArgs {
   int B, T, H, D, K, P, NG, has_r;
@@ -651,6 +653,78 @@ void launch_prologue_bwd(const ProBwdArgs& a, unsigned nblk, int gthr, int nthr,
 }  // namespace atlas
 
 using namespace atlas;
+
+namespace atlas {
+namespace {
+
+// y = x / sqrt(mean(x^2) + 1e-6) over rows of C elements, in fp32, rounded to
+// the dtype once (memory_layer.py:211-216).  Bound by its launch for a prompt
+// and by memory for long rows: one wave per row, 16 bytes per lane and load,
+// the row read again from the cache for the write.  The separate element-wise
+// passes were seven launches: bf16 (60, 512) 34 -> 9 us, (8192, 1024)
+// 53 -> 9, (32768, 512) 90 -> 13 (5.1 TB/s).
+template <int DT, int VEC>
+__global__ void __launch_bounds__(RMS_WAVES * WAVE) rms_norm_kernel(long long rows, int C, const void* x, void* y) {
+  const long long row = (long long)blockIdx.x * RMS_WAVES + wave_id();
+  if (row >= rows) return;
+  using T = std::conditional_t<DT == ATLAS_DTYPE_F32, float, unsigned short>;
+  typedef T vec __attribute__((ext_vector_type(VEC)));
+  const T* xr = static_cast<const T*>(x) + row * C;
+  T* yr = static_cast<T*>(y) + row * C;
+  float sq = 0.f;
+#pragma unroll 4
+  for (int i = lane_id() * VEC; i < C; i += WAVE * VEC) {
+    const vec v = *reinterpret_cast<const vec*>(xr + i);
+#pragma unroll
+    for (int j = 0; j < VEC; ++j) {
+      const T e = v[j];
+      const float f = load_any(&e, 0, DT);
+      sq = fmaf(f, f, sq);
+    }
+  }
+  const float r = rsqrtf(wave_sum(sq) / (float)C + 1e-6f);
+#pragma unroll 4
+  for (int i = lane_id() * VEC; i < C; i += WAVE * VEC) {
+    const vec v = *reinterpret_cast<const vec*>(xr + i);
+    vec o;
+#pragma unroll
+    for (int j = 0; j < VEC; ++j) {
+      const T e = v[j];
+      T z;
+      store_any(&z, 0, DT, load_any(&e, 0, DT) * r);
+      o[j] = z;
+    }
+    *reinterpret_cast<vec*>(yr + i) = o;
+  }
+}
+
+template <int DT>
+void launch_rms_norm(long long rows, int C, const void* x, void* y, hipStream_t st) {
+  constexpr int VEC = DT == ATLAS_DTYPE_F32 ? 4 : 8;
+  const dim3 grid((unsigned)((rows + RMS_WAVES - 1) / RMS_WAVES)), block(RMS_WAVES * WAVE);
+  // 16-byte accesses where every row starts on one, else element by element
+  const bool vec = C % VEC == 0 && ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(y)) & 15) == 0;
+  if (vec) hipLaunchKernelGGL((rms_norm_kernel<DT, VEC>), grid, block, 0, st, rows, C, x, y);
+  else hipLaunchKernelGGL((rms_norm_kernel<DT, 1>), grid, block, 0, st, rows, C, x, y);
+}
+
+}  // namespace
+}  // namespace atlas
+
+extern "C" atlas_status atlas_rms_norm(int64_t rows, int32_t C, const void* x, void* y, int32_t dtype, void* stream) {
+  clear_error();
+  if (rows < 0 || C < 1) return fail(ATLAS_ERR_INVALID_ARGUMENT, "rows %lld, C %d", (long long)rows, C);
+  if (dtype < 0 || dtype > 2) return fail(ATLAS_ERR_INVALID_ARGUMENT, "bad dtype");
+  if (rows == 0) return ATLAS_OK;
+  if (!x || !y) return fail(ATLAS_ERR_INVALID_ARGUMENT, "null pointer");
+  if ((rows + RMS_WAVES - 1) / RMS_WAVES > 0x7fffffffLL) return fail(ATLAS_ERR_UNSUPPORTED_SHAPE, "too many rows");
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  if (dtype == ATLAS_DTYPE_F32) launch_rms_norm<ATLAS_DTYPE_F32>(rows, C, x, y, st);
+  else if (dtype == ATLAS_DTYPE_BF16) launch_rms_norm<ATLAS_DTYPE_BF16>(rows, C, x, y, st);
+  else launch_rms_norm<ATLAS_DTYPE_F16>(rows, C, x, y, st);
+  const hipError_t e = hipGetLastError();
+  return e == hipSuccess ? ATLAS_OK : fail_hip(e, "rms_norm launch");
+}
 
 extern "C" atlas_status atlas_layer_prologue(int32_t B, int32_t T, int32_t H, int32_t D, int32_t conv_kernel,
                                              int32_t poly_degree, int32_t n_gates, int32_t has_retrieve,

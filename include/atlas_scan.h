@@ -235,6 +235,11 @@ atlas_status atlas_linear_scan_bwd(int32_t B, int32_t T, int32_t H, int64_t N,
                                    float* d_gates, float* d_inputs, void* workspace,
                                    size_t workspace_bytes, void* stream);
 
+/* y = x / sqrt(mean(x^2) + 1e-6) over `rows` dense rows of C elements
+ * (atlas_jax/memory_layer.py:211-216): fp32 arithmetic, x and y of dtype. */
+atlas_status atlas_rms_norm(int64_t rows, int32_t C, const void* x, void* y,
+                            int32_t dtype, void* stream);
+
 /* Memory-layer prologue after the input projections: the part of
  * AtlasMemoryLayer.__call__ between the projections and the chunk loop
  * (atlas_jax/memory_layer.py:606-633): causal depthwise convolutions of q, k,

@@ -298,3 +298,29 @@ def test_layer_prologue_paths(dtype, H, D, K, ld_extra, T):
         grads = _layer_prologue_bwd_hip(wide, cw, cb, pc, gb, meta, *cts, dproj_dtype=dt)
         for i, (a, b) in enumerate(zip(grads, want)):
             assert a.shape == b.shape and rel(a, b) <= (1e-5 if i or dt == torch.float32 else one), (i, dt)
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16", "float16"])
+@pytest.mark.parametrize("shape", [(1, 1), (3, 7), (5, 512), (2, 3, 520), (9, 513), (1, 4104), (0, 64)])
+def test_rms_norm_rows(dtype, shape):
+    """The fused row norm (16-byte rows, odd rows and bases, one row to several
+    workgroups) against fp64: one rounding of the dtype and an fp32 sum of C
+    terms (C/2 2^-24 at most); a gradient, a vmap and a transposed input take
+    the torch operations with the same values."""
+    torch = _torch()
+    from atlas_amd import rms_norm
+    dt = getattr(torch, dtype)
+    g = torch.Generator(device="cuda").manual_seed(shape[-1])
+    buf = torch.randn(int(np.prod(shape)) + 1, device="cuda", generator=g).to(dt)
+    tol = {"float32": 2.0 ** -23, "bfloat16": 2.0 ** -8, "float16": 2.0 ** -11}[dtype] + shape[-1] * 2.0 ** -25
+    for x in (buf[:-1].view(shape), buf[1:].view(shape)):
+        xd = x.double()
+        want = xd * (xd.pow(2).mean(-1, keepdim=True) + 1e-6).rsqrt()
+        forms = [rms_norm(x), rms_norm(x.clone().requires_grad_(True)).detach(),
+                 rms_norm(x.transpose(0, -2).contiguous().transpose(0, -2)),
+                 rms_norm(x.mT.contiguous().mT)]
+        if shape[0]:
+            forms.append(torch.vmap(rms_norm)(x))
+        for y in forms:
+            assert y.dtype == dt and y.shape == x.shape
+            assert bool(((y.double() - want).abs() <= tol * want.abs() + 2.0 ** -24).all())
