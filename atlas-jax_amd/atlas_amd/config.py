@@ -3,7 +3,7 @@
 Field names, meanings and defaults follow the reference's AtlasConfig
 (atlas_jax/config.py:6-33) so configs carry over unchanged.  Two fields are
 added: `scan_precision` selects the arithmetic of the HIP scan ("f32": fp32
-MFMA throughout; "f16": fp16 MFMA operands with fp32 accumulation and fp32
+accuracy throughout; "f16": fp16 MFMA operands with fp32 accumulation and fp32
 state; None: "f32" for fp32 activations, "f16" otherwise) when no gradient
 is taken, `scan_backward` the training path of the scan ("hip": the
 library's atlas_scan_bwd; "torch": the inner gradient as differentiable

@@ -128,9 +128,6 @@ struct ModeF16 {
   // Accumulation operands (acc += w * T via an identity MFMA) use bf16: fp32's
   // exponent range, so contributions far below fp16's range are not lost.
   using afrag = bf16x8;
-  __device__ __forceinline__ static f32x16 amma(afrag a, afrag b, f32x16 c) {
-    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
-  }
   __device__ __forceinline__ static afrag a_from_c(const f32x16& t, int kb) {
     afrag f;
 #pragma unroll
@@ -178,7 +175,6 @@ struct ModeF32 {
     return (c == kslot(kb, h, 0)) ? 1.f : 0.f;
   }
   using afrag = float;
-  __device__ __forceinline__ static f32x16 amma(afrag a, afrag b, f32x16 c) { return mma(a, b, c); }
   __device__ __forceinline__ static afrag a_from_c(const f32x16& t, int kb) { return t[kb]; }
   __device__ __forceinline__ static afrag a_identity(int kb, int c, int h, float w) {
     return (c == kslot(kb, h, 0)) ? w : 0.f;

@@ -20,7 +20,8 @@
 //        symmetric: their C-layout tiles serve as operands as they are);
 //   X <- a X + B X     computed as X' = a X (fp32, while the B products run)
 //        then X' + (B/a) X', with X''s own C-layout tiles as the B operand.
-// fp32 path (ModeF32): the Gram passes each 32-column block of X through the
+// fp32 path (ModeF32; E = 256 only, the narrower shapes run on split operands,
+// atlas_pe_split.hpp): the Gram passes each 32-column block of X through the
 // wave's private LDS scratch instead.
 #pragma once
 
@@ -543,20 +544,6 @@ __device__ __forceinline__ float polar_express_wave_t(f32x16 (&X)[D / 32][E / 32
     P::apply_sym(X, A, st, xs);
   }
   return kPEtau[ns];
-}
-
-// One matrix per wave.
-template <class M, int D, int E>
-__device__ __forceinline__ void polar_express_wave(f32x16 (&X)[D / 32][E / 32], int ns, float norm_eps,
-                                                   typename M::elem* scr) {
-  using P = PEWave<M, D, E>;
-  const float ss = P::sumsq(X);
-  P::scale(X, 1.f / (sqrtf(ss + norm_eps) * 1.01f + 1e-6f));
-  for (int st = 0; st < ns; ++st) {
-    f32x16 A[D / 32][D / 32];
-    P::gram(X, A, scr);
-    P::apply(X, A, st);
-  }
 }
 
 // One D x 2EH matrix split by columns over a pair of waves of the same

@@ -23,7 +23,7 @@
 // Y_1 .. Y_{ns-3} go to the workgroup's global scratch, Y_{ns-2} stays in
 // registers, Y_0 is X / nrm again.
 //
-// 4 096 matrices of 64 x 128, 5 steps: 2908 -> 760 us against fp32 MFMA on
+// 4 096 matrices of 64 x 128, 5 steps: 2908 -> 640 us against fp32 MFMA on
 // element-wise LDS operands (one workgroup per CU; the split tiles leave room
 // for two), 2 048 of 64 x 256: 7.2 -> 0.79 ms.  About 1000 products of 32
 // cycles per SIMD and matrix; the barriers between the phases, with waves idle

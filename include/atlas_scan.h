@@ -69,7 +69,8 @@ typedef enum {
 } atlas_dtype;
 
 /* Arithmetic of the matrix-core work inside the scan.
- *   ATLAS_COMPUTE_F32: fp32 MFMA everywhere (parity mode, ~1e-6 per chunk).
+ *   ATLAS_COMPUTE_F32: fp32 accuracy (parity mode, ~1e-6 per chunk): fp32 MFMA,
+ *     and Polar-Express on fp32 operands split into two scaled fp16 parts.
  *   ATLAS_COMPUTE_F16: inner-gradient GEMMs in fp32 MFMA; momentum assembly,
  *     Polar-Express and read-out products with fp16 MFMA operands, fp32
  *     accumulation and fp32 master copies (~2e-3 per chunk). */
@@ -201,7 +202,7 @@ atlas_status atlas_pe_batched(int64_t n, int32_t d1, int32_t d2,
  * row-major fp32 matrices: G holds the cotangent of PE(X) on entry and
  * dPE/dX^T G on return.  min(d1, d2) 32 with max 32/64/128, or 64 with
  * 64/128/256.  compute: ATLAS_COMPUTE_F32
- * (fp32 matrix-core operands) or ATLAS_COMPUTE_F16 (fp16 operands, each
+ * (fp32 operands, each split into two scaled fp16 parts) or ATLAS_COMPUTE_F16 (fp16 operands, each
  * scaled by a power of two, fp32 accumulation).  Workspace:
  * atlas_pe_vjp_workspace_size bytes (0 = unsupported; enough for either
  * compute mode).  X, G and the workspace 16-byte aligned. */
