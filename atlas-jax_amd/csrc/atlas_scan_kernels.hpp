@@ -360,16 +360,19 @@ prep_kernel(ScanArgs p) {
 // coef: gate-only tables of the chunks [c0, c0 + nwin) (independent of the
 // memory state, so a whole window of chunks is computed in parallel, ahead of
 // the chunk loop reaching it).  Grid: streams * nwin.
-// Row t of the chunk is owned by thread t (cs <= CS_MAX; the block holds cs
-// rounded up to whole waves).  The two cs x (cs+1) tables are sized by the
-// runtime cs (coef_lds_bytes(cs)), so at cs = 64 four blocks share a CU.
-// Bound by one wave's chain of LDS reads: cs = 64, 64 blocks, 19 us (33 us with
-// per-thread ranges, which wait for every read, and a division per element).
+// The block holds cs rounded up to whole waves, twice: in the first half thread
+// t owns row t of the window sums (cs <= CS_MAX), in the second half thread s
+// owns column s of the decays a(s->t), which depend on nothing the first half
+// does.  The two cs x (cs+1) tables are sized by the runtime cs
+// (coef_lds_bytes(cs)), so at cs = 64 four blocks share a CU.
+// Bound by one wave's chain of LDS reads: cs = 64, 64 blocks, 14 us (19 us with
+// the decays after the window sums in the same threads; 33 us with per-thread
+// ranges, which wait for every read, and a division per element).
 //   c[t,i] = (2/D) g'_i sum_{s=i}^{min(t,i+w-1)} theta(s->t) (-eta_s),
 //   evaluated as g'_i (R_t[i] - R_t[i+w]) with suffix sums
 //   R_t[s] = sum_{u=s}^{t} theta(u->t) (-eta_u).
 // ===========================================================================
-__global__ void __launch_bounds__(CS_MAX)
+__global__ void __launch_bounds__(2 * CS_MAX)
 coef_kernel(ScanArgs p, int c0, int nwin) {
   extern __shared__ float cl[];
   const int cs = p.cs, CP = cs + 1;
@@ -382,36 +385,41 @@ coef_kernel(ScanArgs p, int c0, int nwin) {
   float* C = R + cs * CP;        // [cs][CP]
   const int stream = blockIdx.x / nwin, chunk = c0 + blockIdx.x % nwin;
   const int b = stream / p.H, hh = stream % p.H;
-  const int t = threadIdx.x;
-  if (t < cs) {
+  const int half = blockDim.x / 2;
+  const bool sums = (int)threadIdx.x < half;   // whole waves
+  const int t = sums ? threadIdx.x : threadIdx.x - half;
+  if (sums && t < cs) {
     const Gates G = load_gates(p, b, hh, chunk * cs + t);
     ga[t] = G.a; ge[t] = G.e; gt[t] = G.th; gg[t] = G.g;
   }
   __syncthreads();
   const long long tb = chunk_table(p, stream, chunk);
+  float* cmt = p.cmt + tb * cs * cs;
   // Every loop below runs over the same tokens in every thread (a thread's own
   // range is a predicate) in steps of four (cs is a multiple of 4), whose reads
   // are all issued before their first use.
-  const bool row = t < cs;
-  float* Rt = R + (row ? t : 0) * CP;
-  float* Ct = C + (row ? t : 0) * CP;
-  {
-    float th = 1.f, apv = 1.f;
+  const bool row = sums && t < cs;
+  if (!sums && t < cs) {   // a(t->r) for every row r, and the prefixes of theta and alpha up to t
+    float* am = p.am + tb * cs * cs + t;
+    float th = 1.f, apv = 1.f, prod = 1.f;
     for (int r0 = 0; r0 < cs; r0 += 4) {
       float g1[4], g2[4];
 #pragma unroll
       for (int u = 0; u < 4; ++u) { g1[u] = gt[r0 + u]; g2[u] = ga[r0 + u]; }
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
-        th = r0 + u <= t ? th * g1[u] : th;
-        apv = r0 + u <= t ? apv * g2[u] : apv;
+        const int r = r0 + u;
+        th = r <= t ? th * g1[u] : th;
+        apv = r <= t ? apv * g2[u] : apv;
+        prod = r > t ? prod * g2[u] : 1.f;
+        am[(long long)r * cs] = r >= t ? prod : 0.f;
       }
     }
-    if (row) {
-      p.thp[tb * cs + t] = th;
-      p.ap[tb * cs + t] = apv;
-    }
+    p.thp[tb * cs + t] = th;
+    p.ap[tb * cs + t] = apv;
   }
+  float* Rt = R + (row ? t : 0) * CP;
+  float* Ct = C + (row ? t : 0) * CP;
   // Window sums sum_{s=i}^{min(t, i+w-1)} m_t[s], m_t[s] = theta(s->t)
   // (-eta_s) (0 past t), without subtraction: over blocks of w tokens, the
   // in-block suffix sums (into Rt) and prefix sums (into Ct); a window is
@@ -479,44 +487,26 @@ coef_kernel(ScanArgs p, int c0, int nwin) {
     m = (m > 0.f) ? m : 1.f;
     mr[t] = m;
     p.cm[tb * cs + t] = m;
-    // a(s->t) row t into Ct (the prefix sums are no longer needed)
-    float prod = 1.f;
-    for (int s0 = cs - 4; s0 >= 0; s0 -= 4) {
-      float g1[4];
-#pragma unroll
-      for (int u = 0; u < 4; ++u) g1[u] = ga[min(s0 + u + 1, cs - 1)];
-#pragma unroll
-      for (int u = 3; u >= 0; --u) {
-        const int s = s0 + u;
-        prod = s < t ? prod * g1[u] : 1.f;
-        Ct[s] = s <= t ? prod : 0.f;
-      }
-    }
   }
   __syncthreads();
-  // column t of every row
-  float* cmt = p.cmt + tb * cs * cs;
-  float* am = p.am + tb * cs * cs;
-  if (row) {
-    for (int r0 = 0; r0 < cs; r0 += 4) {
-      float c1[4], m1[4], a1[4];
+  // column t of every row, the rows split over the two halves
+  if (t < cs) {
+    const int lo = sums ? 0 : (cs / 8) * 4, hi = sums ? (cs / 8) * 4 : cs;
+    for (int r0 = lo; r0 < hi; r0 += 4) {
+      float c1[4], m1[4];
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
         c1[u] = R[(r0 + u) * CP + t];
         m1[u] = mr[r0 + u];
-        a1[u] = C[(r0 + u) * CP + t];
       }
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        cmt[(r0 + u) * cs + t] = c1[u] / m1[u];
-        am[(r0 + u) * cs + t] = a1[u];
-      }
+      for (int u = 0; u < 4; ++u) cmt[(r0 + u) * cs + t] = c1[u] / m1[u];
     }
   }
 }
 
 constexpr size_t coef_lds_bytes(int cs = CS_MAX) { return sizeof(float) * (size_t)(5 * CS_MAX + 2 * cs * (cs + 1)); }
-inline dim3 coef_block(int cs) { return dim3(((cs + 63) / 64) * 64); }
+inline dim3 coef_block(int cs) { return dim3(2 * ((cs + 63) / 64) * 64); }
 
 template <int D, int E>
 constexpr size_t prep_lds_bytes() {
