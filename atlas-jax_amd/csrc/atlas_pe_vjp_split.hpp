@@ -17,8 +17,9 @@
 //   3  B and C shared the same way; every wave updates its own blocks, whose
 //      C tiles are the B operands as they are.
 // The forward recompute has the same phases with one upper tile of A and B per
-// wave.  G is scaled by a power of two per step that brings its largest entry
-// into [1, 2); with |Y| <= 2 (|A| <= 4, |Gs| <= 1024, |C| < 2^15 for the sizes
+// wave.  G is brought to a largest entry in [1, 2) by a power of two before the
+// first step and back after the normalisation (cotangents of any size,
+// subnormal ones included), and again for each step's operands; with |Y| <= 2 (|A| <= 4, |Gs| <= 1024, |C| < 2^15 for the sizes
 // compiled) fixed powers of two keep every operand in fp16's range.
 // Y_1 .. Y_{ns-3} go to the workgroup's global scratch, Y_{ns-2} stays in
 // registers, Y_0 is X / nrm again.
@@ -55,6 +56,9 @@ struct VjpSplit {
   // scratch floats of one workgroup
   static constexpr size_t scratch_floats(int ns) { return ns > 3 ? (size_t)(ns - 3) * D * E : 0; }
 };
+
+// e with 2^e m in [1, 2) (0 for 0, infinities and NaN)
+__device__ __forceinline__ int vjp_exponent(float m) { return m > 0.f && m < INFINITY ? -ilogbf(m) : 0; }
 
 template <int D, int E>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(VjpSplit<D, E>::PER_CU)))
@@ -184,6 +188,28 @@ pe_vjp_split_kernel(long long n, int ns, int tall, const float* X, float* G, flo
         P::put_block(b, 0, s, st + (w + 4 * q) * V::BLK, l);
       }
   };
+  auto scale2 = [&](Tiles& t, int e) {   // times 2^e
+#pragma unroll
+    for (int q = 0; q < BPW; ++q)
+#pragma unroll
+      for (int I = 0; I < TI; ++I)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) t[q][I][r] = __builtin_amdgcn_ldexpf(t[q][I][r], e);
+  };
+  // the block's largest |t|, through red[8 ..] (a barrier: every wave's earlier LDS accesses are done)
+  auto block_max4 = [&](const Tiles& t) {
+    float mx = 0.f;
+#pragma unroll
+    for (int q = 0; q < BPW; ++q)
+#pragma unroll
+      for (int I = 0; I < TI; ++I)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) mx = fmaxf(mx, own(q) ? fabsf(t[q][I][r]) : 0.f);
+    mx = wave_max(mx);
+    if (lane == 0) red[8 + w] = mx;
+    __syncthreads();
+    return fmaxf(fmaxf(red[8], red[9]), fmaxf(red[10], red[11]));
+  };
   auto block_sum4 = [&](float x, int slot) {   // fixed order; slot: 4 floats of red
     x = wave_sum(x);
     if (lane == 0) red[slot + w] = x;
@@ -267,7 +293,12 @@ pe_vjp_split_kernel(long long n, int ns, int tall, const float* X, float* G, flo
     }
 
     // ---- backward through the steps
+    // G is brought to a largest entry in [1, 2) before the first step and back
+    // after the normalisation: its own size may be any, subnormal included.
     load(Gb, Gm);
+    const int eg = vjp_exponent(block_max4(Gb));
+    scale2(Gb, eg);
+    __syncthreads();   // red is written again
     for (int k = ns - 1; k >= 0; --k) {
       if (k + 1 < ns) {
         if (k == 0) {
@@ -296,17 +327,7 @@ pe_vjp_split_kernel(long long n, int ns, int tall, const float* X, float* G, flo
                 }
         }
       }
-      float mx = 0.f;
-#pragma unroll
-      for (int q = 0; q < BPW; ++q)
-#pragma unroll
-        for (int I = 0; I < TI; ++I)
-#pragma unroll
-          for (int r = 0; r < 16; ++r) mx = fmaxf(mx, own(q) ? fabsf(Gb[q][I][r]) : 0.f);
-      mx = wave_max(mx);
-      if (lane == 0) red[8 + w] = mx;
-      __syncthreads();   // also: the previous step's B and C have been read
-      const float sg = pow2_scale(fmaxf(fmaxf(red[8], red[9]), fmaxf(red[10], red[11]))), isg = 1.f / sg;
+      const float sg = pow2_scale(block_max4(Gb)), isg = 1.f / sg;   // (its barrier: the previous step's B and C have been read)
       const float ka = kPE[k][0], kb_ = kPE[k][1], kc = kPE[k][2];
       stage(yst, Y, YS);
       stage(gst, Gb, sg * GS);
@@ -392,7 +413,9 @@ pe_vjp_split_kernel(long long n, int ns, int tall, const float* X, float* G, flo
         const int e = 32 * (w + 4 * q) + c;
 #pragma unroll
         for (int I = 0; I < TI; ++I) {
-          const f32x16 d = Gb[q][I] * inv - coef * Y[q][I];
+          f32x16 d = Gb[q][I] * inv - coef * Y[q][I];
+#pragma unroll
+          for (int r = 0; r < 16; ++r) d[r] = __builtin_amdgcn_ldexpf(d[r], -eg);
           if (tall) {
 #pragma unroll
             for (int g = 0; g < 4; ++g)

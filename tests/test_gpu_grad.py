@@ -363,3 +363,36 @@ def test_non_default_stream_bitwise(train_precision):
     torch.cuda.synchronize()
     for i, (a, b) in enumerate(zip(got, ref)):
         assert torch.equal(a, b), f"output {i} differs between the default and a side stream"
+
+
+@pytest.mark.parametrize("E", [64, 128])
+def test_training_gradients_of_a_masked_prompt(E):
+    """A loss on the last tokens only: through the tokens before them the
+    cotangents of Polar-Express shrink by alpha (about 0.15) a token, below
+    every normal number.  All gradients are finite, and as close to the
+    float64 oracle as those of the torch-composed backward, which forms the
+    same products in fp32 (four times its error, or 1e-4)."""
+    torch = _torch()
+    from atlas_amd import DeepMemoryState, memory_scan
+    g = torch.Generator().manual_seed(E)
+    B, T, H, D, cs = 1, 64, 1, 64 if E == 128 else 32, 64
+    rnd = lambda *s: torch.randn(*s, generator=g, dtype=torch.float64)  # noqa: E731
+    q, k, v = (x / x.norm(dim=-1, keepdim=True) for x in (rnd(B, T, H, D), rnd(B, T, H, D), rnd(B, T, H, D)))
+    al, et, th, ga = (torch.sigmoid(0.2 * rnd(B, T, H) + b) for b in (-1.75, -2.0, 0.0, 0.0))
+    st = [rnd(B, H, D, E) / 8, rnd(B, H, E, D) / 8, 0.05 * rnd(B, H, D, E), 0.05 * rnd(B, H, E, D)]
+    f64 = [t.float().double() for t in (q, k, v, al, et, th, ga, *st)]
+    dy = rnd(B, T, H, D)
+    dy[:, :T - 4] = 0
+    xs = [t.clone().requires_grad_(True) for t in f64]
+    y_r, _ = RT.memory_scan_t(*xs[:7], tuple(xs[7:]), cs, 16, 5, False)
+    ref = torch.autograd.grad(y_r, xs, dy, allow_unused=True)
+    err = {}
+    for how in ("hip", "torch"):
+        gi = [t.float().cuda().requires_grad_(True) for t in f64]
+        y, _ = memory_scan(*gi[:7], DeepMemoryState(*gi[7:]), cs, 16, 5, precision="f32", backward=how)
+        got = torch.autograd.grad(y, gi, dy.float().cuda())
+        assert all(bool(torch.isfinite(t).all()) for t in got), how
+        err[how] = [SC.rel_l2(a.double().cpu().numpy(), b.numpy()) for a, b in zip(got, ref)]
+    print(f"masked prompt E{E}: hip {err['hip']}, torch {err['torch']}", flush=True)
+    for i, (a, b) in enumerate(zip(err["hip"], err["torch"])):
+        assert a <= max(1e-4, 4 * b), i

@@ -303,3 +303,23 @@ def test_pe_vjp_f32_split_accuracy(d1, d2, steps, n, gscale):
     e = rel(polar_express_vjp(X, C, steps)[sel])
     print(f"split VJP {d1}x{d2} ns{steps} n={n} G {gscale:g}: {e:.2e} (bar {bar:.2e})", flush=True)
     assert e <= bar
+
+
+@pytest.mark.parametrize("d1,d2", [(32, 32), (64, 128), (128, 64), (64, 256)])
+@pytest.mark.parametrize("exp", [-139, -126, -118, -114, -100, 110])
+def test_pe_vjp_f32_cotangent_range(d1, d2, exp):
+    """fp32 VJP for cotangents of size 2^exp, subnormal ones included.  The VJP
+    is linear in them and scales them by powers of two, so the result is 2^exp
+    times that of cotangents of size one, each element rounded once more where
+    it is subnormal (by half of 2^-149)."""
+    torch = _torch()
+    from atlas_amd.autograd import polar_express_vjp
+    g = torch.Generator(device="cuda").manual_seed(d1 + 3 * d2)
+    X = torch.randn(5, d1, d2, device="cuda", generator=g)
+    C = (torch.randn(5, d1, d2, device="cuda", generator=g) * 256).round().clamp(-1000, 1000) / 256   # exact at 2^-139
+    unit = polar_express_vjp(X, C, 5).double()
+    got = polar_express_vjp(X, C * 2.0 ** exp, 5)
+    assert bool(torch.isfinite(got).all())
+    err = (got.double() * 2.0 ** -exp - unit).abs().max()
+    print(f"VJP {d1}x{d2} G 2^{exp}: largest error {float(err):.2e}, half a unit {2.0 ** (-150 - exp):.2e}", flush=True)
+    assert err <= 2.0 ** (-150 - exp)
