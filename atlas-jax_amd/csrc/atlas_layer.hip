@@ -635,18 +635,24 @@ __global__ void __launch_bounds__(256) prologue_bwd_reduce_kernel(const float* p
   else dp[i - n_w - n_b - n_g] = s;
 }
 
+// (up to 69 KiB of LDS, at 256 threads to a group and four taps: the limit is
+// raised as for every launch that may pass 64 KiB)
 template <int K>
-void launch_prologue_bwd(const ProBwdArgs& a, unsigned nblk, int gthr, int nthr, bool aligned, hipStream_t st) {
+hipError_t launch_prologue_bwd(const ProBwdArgs& a, unsigned nblk, int gthr, int nthr, bool aligned, hipStream_t st) {
   const int G = std::min(512 / gthr, PRO_BR / 4);
   const size_t lds = (size_t)gthr * (12 * K + 12 + 9) * sizeof(float);
   auto go = [&](void (*k)(ProBwdArgs, int, int, int)) {
+    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(k),
+                                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    if (e != hipSuccess) return e;
     hipLaunchKernelGGL(k, dim3(nblk), dim3(G * gthr), lds, st, a, nthr, gthr, G);
+    return hipGetLastError();
   };
   const int dt = K == 4 && aligned && a.f.proj_dtype == a.gdt && a.f.proj_dtype == a.ddt ? a.gdt : -1;
-  if (dt == 0) go(prologue_bwd_kernel<K, K == 4 ? 0 : -1>);
-  else if (dt == 1) go(prologue_bwd_kernel<K, K == 4 ? 1 : -1>);
-  else if (dt == 2) go(prologue_bwd_kernel<K, K == 4 ? 2 : -1>);
-  else go(prologue_bwd_kernel<K, -1>);
+  if (dt == 0) return go(prologue_bwd_kernel<K, K == 4 ? 0 : -1>);
+  if (dt == 1) return go(prologue_bwd_kernel<K, K == 4 ? 1 : -1>);
+  if (dt == 2) return go(prologue_bwd_kernel<K, K == 4 ? 2 : -1>);
+  return go(prologue_bwd_kernel<K, -1>);
 }
 
 }  // namespace
@@ -847,15 +853,17 @@ extern "C" atlas_status atlas_layer_prologue_bwd_as(
   if (nblk > 0x7fffffffLL) return fail(ATLAS_ERR_UNSUPPORTED_SHAPE, "too many token rows");
   hipStream_t st = static_cast<hipStream_t>(stream);
   const bool aligned = proj_ld % 4 == 0 && dproj_ld % 4 == 0 && !mis(proj, 4 * esz) && !mis(dproj, 4 * dsz);
+  hipError_t e;
   switch (conv_kernel) {
-    case 1: launch_prologue_bwd<1>(a, (unsigned)nblk, threads, nthr, aligned, st); break;
-    case 2: launch_prologue_bwd<2>(a, (unsigned)nblk, threads, nthr, aligned, st); break;
-    case 3: launch_prologue_bwd<3>(a, (unsigned)nblk, threads, nthr, aligned, st); break;
-    default: launch_prologue_bwd<4>(a, (unsigned)nblk, threads, nthr, aligned, st); break;
+    case 1: e = launch_prologue_bwd<1>(a, (unsigned)nblk, threads, nthr, aligned, st); break;
+    case 2: e = launch_prologue_bwd<2>(a, (unsigned)nblk, threads, nthr, aligned, st); break;
+    case 3: e = launch_prologue_bwd<3>(a, (unsigned)nblk, threads, nthr, aligned, st); break;
+    default: e = launch_prologue_bwd<4>(a, (unsigned)nblk, threads, nthr, aligned, st); break;
   }
+  if (e != hipSuccess) return fail_hip(e, "prologue backward launch");
   hipLaunchKernelGGL(prologue_bwd_reduce_kernel, dim3((unsigned)((a.part_len + 31) / 32)), dim3(256), 0, st,
                      a.part, (int)nblk, a.part_len, n_w, n_b, n_g, d_conv_w, d_conv_b, d_gate_b, d_poly);
-  const hipError_t e = hipGetLastError();
+  e = hipGetLastError();
   return e == hipSuccess ? ATLAS_OK : fail_hip(e, "prologue backward launch");
 }
 

@@ -265,11 +265,14 @@ def test_layer_prologue_backward(dtype, poly, H, D, K, n_gates, has_r, T):
 
 @pytest.mark.parametrize("dtype,H,D,K,ld_extra,T", [("bf16", 8, 64, 4, 0, 63), ("f16", 12, 64, 4, 0, 129),
                                                     ("f32", 4, 32, 4, 0, 5), ("bf16", 8, 64, 4, 1, 66),
-                                                    ("bf16", 5, 16, 4, 0, 64), ("f32", 16, 64, 3, 0, 70)])
+                                                    ("bf16", 5, 16, 4, 0, 64), ("f32", 16, 64, 3, 0, 70),
+                                                    ("f32", 16, 64, 4, 0, 70), ("bf16", 16, 64, 4, 0, 70),
+                                                    ("f16", 16, 64, 4, 2, 65)])
 def test_layer_prologue_paths(dtype, H, D, K, ld_extra, T):
     """The prologue's forward and backward on every load path (rows aligned to
     four elements in each dtype, a row stride that is not, conv kernels below
-    4, one to eight groups of threads, runs that end mid-block) against the
+    4, one to eight groups of threads, more than 64 KiB of LDS (1024 channels,
+    four taps), runs that end mid-block) against the
     same arithmetic in torch (layer_prologue_reference_ops, fp32) and its
     autograd: the 16-bit outputs within one rounding (2^-8 bf16, 2^-11 fp16),
     fp32 sums of up to 2 T terms within 1e-5."""
