@@ -194,7 +194,7 @@ __device__ __forceinline__ void load_frags(const SwaArgs& a, const void* x, long
 // (four per score: multiply-add, exp, sum, half a conversion and half a
 // maximum; 32 exps at a quarter of the rate; the rotation and conversion of the
 // staged keys) against 16 products, 63 % VALU-busy and 26 % MFMA-busy at a
-// clock of 1.9 GHz (power).  B4 T16384 H12, window 2048, bf16: 631 us, 0.65
+// clock of 1.9 GHz (power).  B4 T16384 H12, window 2048, bf16: 654 us, 0.63
 // PFLOP/s; 1853 us when every block was loaded, rotated, transposed with 2-byte
 // LDS writes and used between two barriers, 128 queries to a workgroup.  A
 // wave per SIMD more (four, spilling 19-35 registers) takes 905-1320 us, 32
@@ -212,7 +212,7 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(QT
   const int bh = lb / nqb, qb = lb % nqb;
   const int b = bh / a.H, hh = bh % a.H;
   const int tid = threadIdx.x, lane = lane_id(), c = lane & 31, h = lane >> 5, w = wave_id();
-  const int q0 = qb * BQ, qw = q0 + 32 * QT * w;
+  const int q0 = qb * BQ, qw = q0 + 32 * QT * w, qs = __builtin_amdgcn_readfirstlane(qw);
   const long long base_bh = (long long)b * a.sb + (long long)hh * a.sh;
 
   frag qf[QT][4];
@@ -336,16 +336,27 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(QT
         }
         l[t] += ps;
       }
+      // A 32 x 32 tile that no query of it sees into is left out (its
+      // probabilities are zeros, but 0 times an infinite value is not).  The
+      // branches cost 3 % of the 512-query form (two copies of the products, one
+      // without branches, spill 15-108 registers and take 1.5 to 2 times as long).
 #pragma unroll
-      for (int kt = 0; kt < 2; ++kt)
+      for (int kt = 0; kt < 2; ++kt) {
+        frag vf[2][2];
 #pragma unroll
         for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
-          for (int I = 0; I < 2; ++I) {
-            const frag vf = ld_tr(Vs[buf], tr, I, kt, kb);
+          for (int I = 0; I < 2; ++I) vf[kb][I] = ld_tr(Vs[buf], tr, I, kt, kb);
 #pragma unroll
-            for (int t = 0; t < QT; ++t) O[t][I] = M::mma(vf, pf[t][kt][kb], O[t][I]);
-          }
+        for (int t = 0; t < QT; ++t) {
+          const int k0 = kb0 + 32 * kt, q32 = qs + 32 * t;
+          if (k0 > q32 + 31 || k0 + 31 < q32 - a.window) continue;
+#pragma unroll
+          for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+            for (int I = 0; I < 2; ++I) O[t][I] = M::mma(vf[kb][I], pf[t][kt][kb], O[t][I]);
+        }
+      }
     }
     if (more) stage(buf ^ 1);
     __syncthreads();

@@ -366,3 +366,31 @@ def test_swa_backward_grad_dtype(dtype, T, window):
     for a, b in zip(full, half):
         ulp = a.abs() * torch.finfo(tdt).eps + torch.finfo(tdt).smallest_normal * torch.finfo(tdt).eps
         assert b.dtype == tdt and bool(((a.to(tdt).float() - b.float()).abs() <= ulp).all())
+
+
+@pytest.mark.parametrize("dtype", ["bf16", "f16"])
+@pytest.mark.parametrize("B,T,H,window", [(1, 300, 2, 70), (1, 130, 1, 4096), (1, 257, 1, 0),
+                                          (1, 8200, 48, 2048)])   # the last on 512-query workgroups
+def test_swa_nonfinite_values_stay_in_their_tile(dtype, B, T, H, window):
+    """An infinite or NaN value row reaches the queries that see it and no
+    query outside the 32-query tiles with one that sees its 32-key tile (a
+    masked key's probability is 0, and 0 times infinity is NaN): those are
+    bit for bit what they are with finite values."""
+    torch = _torch()
+    from atlas_amd import RotaryEmbedding, swa_attention
+    tdt = torch.bfloat16 if dtype == "bf16" else torch.float16
+    g = torch.Generator(device="cuda").manual_seed(T)
+    qkv = torch.randn(B, T, 3, H, 64, device="cuda", generator=g).to(tdt)
+    cos, sin = RotaryEmbedding(64)(T)
+    clean = swa_attention(*qkv.unbind(2), window, cos, sin)
+    t = torch.arange(T, device="cuda")
+    for s in (0, 33, 95, T // 2 + 5, T - 1) if T < 4096 else (95, T // 2 + 5):
+        sees = (s <= t) & (t - s <= window)
+        s0, t0 = s // 32 * 32, t // 32 * 32
+        reach = (s0 <= t0 + 31) & (s0 + 31 >= t0 - window)
+        for bad in (float("inf"), float("nan")):
+            x = qkv.clone()
+            x[:, s, 2] = bad
+            out = swa_attention(*x.unbind(2), window, cos, sin)
+            assert torch.equal(out[:, ~reach], clean[:, ~reach]), (s, bad)
+            assert not bool(torch.isfinite(out[:, sees]).any()), (s, bad)
