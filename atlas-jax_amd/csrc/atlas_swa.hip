@@ -704,16 +704,20 @@ void swa_launch_fwd_as(const SwaArgs& a, hipStream_t st) {
 }
 
 // 512 queries per workgroup rotate and convert each key a quarter as often as
-// 128 do, but stage up to 7 blocks that a wave of a narrow band skips, and fill
-// the CUs more coarsely.  They are the faster choice where the band is wide
-// and every CU gets at least three workgroups (us, 128 / 512 queries; B4 H12
-// T16384: window 512 297 / 307, 1024 445 / 424, 2048 717 / 645, 4096 1197 / 1061;
-// window 2048 with two workgroups per CU, B1 H12 T16384: 203 / 202, B4 H12
-// T4096: 172 / 181).
+// 128 do, but stage up to 7 blocks that a wave of a narrow band skips (and, over
+// the first `window` queries, up to 7 of the few there are), and fill the CUs
+// more coarsely.  They are the faster choice where the sequence is long, the
+// band wide and every CU gets at least three workgroups.  us, 128 / 512
+// queries, H12: window 1024 at B12 T8192 617 / 624, B8 T12288 662 / 644, B6
+// T16384 670 / 657; window 1536 at B24 T4096 714 / 779, B16 T6144 786 / 783, B12
+// T8192 820 / 791, B6 T16384 893 / 816; window 2048 at B24 T4096 840 / 906, B12
+// T8192 1001 / 937, B6 T16384 1096 / 984; window 4096 at B16 T6144 1384 / 1387,
+// B12 T8192 1546 / 1471, B6 T16384 1848 / 1613; window 8192 at B6 T16384 2936 /
+// 2626.  With 384 workgroups, B1 T16384, window 2048: 183 / 209.
 atlas_status swa_launch_fwd(const SwaArgs& a, void* stream) {
   hipStream_t st = static_cast<hipStream_t>(stream);
   const long long n512 = (long long)a.B * a.H * ((a.T + 511) / 512);
-  if (min(a.window, a.T / 2) >= 1024 && n512 >= 3 * 256)
+  if (n512 >= 3 * 256 && a.T >= 8192 && a.window >= (a.T >= 12288 ? 1024 : 1536))
     swa_launch_fwd_as<8, 2>(a, st);
   else
     swa_launch_fwd_as<4, 1>(a, st);
