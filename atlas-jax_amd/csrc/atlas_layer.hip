@@ -121,7 +121,8 @@ __global__ void __launch_bounds__(PRO_WAVES * WAVE) prologue_kernel(ProArgs a) {
 
 // Four consecutive channels on their way from memory: DT 0 fp32, 1 bf16, 2
 // fp16 as loaded (converted where they are used, so that the next token's
-// loads can be in flight); DT -1: any dtype and alignment, converted at once.
+// loads can be in flight); DT -1: any dtype and alignment, converted at once;
+// DT -2: any dtype, as loaded, aligned to the four elements.
 template <int DT>
 struct Quad {
   uint2 w;
@@ -152,6 +153,25 @@ struct Quad<-1> {
   }
   __device__ __forceinline__ f32x4 get() const { return v; }
 };
+template <>
+struct Quad<-2> {
+  f32x4 v;   // (16-bit channels: in the first half)
+  int dt;
+  __device__ __forceinline__ void load(const void* p, int64_t i, int dtype) {
+    dt = dtype;
+    if (dtype == 0) {
+      v = *reinterpret_cast<const f32x4*>(static_cast<const float*>(p) + i);
+    } else {
+      const float2 w = *reinterpret_cast<const float2*>(static_cast<const uint16_t*>(p) + i);
+      v = f32x4{w.x, w.y, 0.f, 0.f};
+    }
+  }
+  __device__ __forceinline__ f32x4 get() const {
+    if (dt == 0) return v;
+    const uint2 w{__float_as_uint(v[0]), __float_as_uint(v[1])};
+    return dt == 1 ? Quad<1>{w}.get() : Quad<2>{w}.get();
+  }
+};
 typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 template <int DT>
 __device__ __forceinline__ void put4(void* p, int64_t i, int dtype, f32x4 x) {
@@ -163,6 +183,8 @@ __device__ __forceinline__ void put4(void* p, int64_t i, int dtype, f32x4 x) {
   else if constexpr (DT == 2)
     *reinterpret_cast<f16x4*>(static_cast<_Float16*>(p) + i) =
         f16x4{(_Float16)x[0], (_Float16)x[1], (_Float16)x[2], (_Float16)x[3]};
+  else if constexpr (DT == -2)
+    store4_any(p, i, dtype, x);
   else
 #pragma unroll
     for (int u = 0; u < 4; ++u) store_any(p, i + u, dtype, x[u]);
@@ -313,14 +335,16 @@ __global__ void __launch_bounds__(256) prologue_vec_kernel(ProArgs a, int nthr) 
   }
 }
 
+// (its loads and stores are all aligned to four elements; the dtype is compiled
+// in where the taps are the default four and it is one for both)
 template <int K>
 void launch_prologue_vec(const ProArgs& a, unsigned blocks, int threads, int nthr, hipStream_t st) {
   auto go = [&](void (*k)(ProArgs, int)) { hipLaunchKernelGGL(k, dim3(blocks), dim3(threads), 0, st, a, nthr); };
-  const int dt = K == 4 && a.proj_dtype == a.out_dtype ? a.proj_dtype : -1;
-  if (dt == 0) go(prologue_vec_kernel<K, K == 4 ? 0 : -1>);
-  else if (dt == 1) go(prologue_vec_kernel<K, K == 4 ? 1 : -1>);
-  else if (dt == 2) go(prologue_vec_kernel<K, K == 4 ? 2 : -1>);
-  else go(prologue_vec_kernel<K, -1>);
+  const int dt = K == 4 && a.proj_dtype == a.out_dtype ? a.proj_dtype : -2;
+  if (dt == 0) go(prologue_vec_kernel<K, K == 4 ? 0 : -2>);
+  else if (dt == 1) go(prologue_vec_kernel<K, K == 4 ? 1 : -2>);
+  else if (dt == 2) go(prologue_vec_kernel<K, K == 4 ? 2 : -2>);
+  else go(prologue_vec_kernel<K, -2>);
 }
 
 // ---- backward ---------------------------------------------------------------

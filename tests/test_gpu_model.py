@@ -303,6 +303,31 @@ def test_layer_prologue_paths(dtype, H, D, K, ld_extra, T):
             assert a.shape == b.shape and rel(a, b) <= (1e-5 if i or dt == torch.float32 else one), (i, dt)
 
 
+@pytest.mark.parametrize("K,proj_dtype,out_dtype", [(1, "bfloat16", "bfloat16"), (2, "float16", "float16"),
+                                                    (3, "bfloat16", "bfloat16"), (4, "float32", "bfloat16"),
+                                                    (4, "float16", "float32"), (3, "bfloat16", "float16")])
+@pytest.mark.parametrize("T", [1, 7])
+def test_layer_prologue_mixed_dtypes(K, proj_dtype, out_dtype, T):
+    """The forward's aligned path with the dtypes at run time (fewer than four
+    taps, or a projection of another dtype than the outputs) against the same
+    arithmetic in torch: one rounding of the outputs' dtype, fp32 gates."""
+    torch = _torch()
+    from atlas_amd.memory_layer import _layer_prologue_hip, layer_prologue_reference_ops
+    pdt, odt = getattr(torch, proj_dtype), getattr(torch, out_dtype)
+    B, H, D = 3, 4, 32
+    g = torch.Generator(device="cuda").manual_seed(K + T)
+    proj = torch.randn(B * T, 3 * H * D + 5 * H, device="cuda", generator=g).to(pdt)
+    cw = torch.randn(3, H * D, K, device="cuda", generator=g) * 0.5
+    cb = torch.randn(3, H * D, device="cuda", generator=g) * 0.1
+    pc, gb = torch.tensor([1.0, 0.5], device="cuda"), torch.randn(4, H, device="cuda", generator=g)
+    got = _layer_prologue_hip(proj, cw, cb, pc, gb, (B, T, H, D, K, 2, 4, True, 0.1, odt))
+    ref = layer_prologue_reference_ops(proj.float(), cw, cb, pc, gb, (B, T, H, D, K, 2, 4, True, 0.1, torch.float32))
+    one = {"float32": 1e-5, "bfloat16": 2.0 ** -8, "float16": 2.0 ** -11}[out_dtype]
+    for i, (a, b) in enumerate(zip(got, ref)):
+        assert a.dtype == (odt if i < 3 else torch.float32)
+        assert float((a.double() - b.double()).norm() / b.double().norm()) <= (one if i < 3 else 1e-5), i
+
+
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16", "float16"])
 @pytest.mark.parametrize("shape", [(1, 1), (3, 7), (5, 512), (2, 3, 520), (9, 513), (1, 4104), (0, 64)])
 def test_rms_norm_rows(dtype, shape):
