@@ -361,9 +361,10 @@ prep_kernel(ScanArgs p) {
 // memory state, so a whole window of chunks is computed in parallel, ahead of
 // the chunk loop reaching it).  Grid: streams * nwin.
 // The block holds cs rounded up to whole waves, twice: in the first half thread
-// t owns row t of the window sums (cs <= CS_MAX), in the second half thread s
-// owns column s of the decays a(s->t), which depend on nothing the first half
-// does.  The two cs x (cs+1) tables are sized by the runtime cs
+// t owns row t of the window sums (cs <= CS_MAX), in the second half row t of
+// the decays a(s->t), which depend on nothing the first half does.  The decays
+// are multiplied from t downwards: another order differs in the last bit, which
+// the recurrence over the chunks amplifies.  The two cs x (cs+1) tables are sized by the runtime cs
 // (coef_lds_bytes(cs)), so at cs = 64 four blocks share a CU.
 // Bound by one wave's chain of LDS reads: cs = 64, 64 blocks, 14 us (19 us with
 // the decays after the window sums in the same threads; 33 us with per-thread
@@ -399,20 +400,31 @@ coef_kernel(ScanArgs p, int c0, int nwin) {
   // range is a predicate) in steps of four (cs is a multiple of 4), whose reads
   // are all issued before their first use.
   const bool row = sums && t < cs;
-  if (!sums && t < cs) {   // a(t->r) for every row r, and the prefixes of theta and alpha up to t
-    float* am = p.am + tb * cs * cs + t;
-    float th = 1.f, apv = 1.f, prod = 1.f;
+  if (!sums && t < cs) {   // a(s->t) = alpha_t alpha_(t-1) .. alpha_(s+1), multiplied in this order, and the prefixes up to t
+    float* am = p.am + (tb * cs + t) * cs;
+    float prod = 1.f;
+    for (int s0 = cs - 4; s0 >= 0; s0 -= 4) {
+      float g1[4];
+      f32x4 o;
+#pragma unroll
+      for (int u = 0; u < 4; ++u) g1[u] = ga[s0 + u + 1];   // (one past the last is not used)
+#pragma unroll
+      for (int u = 3; u >= 0; --u) {
+        const int s = s0 + u;
+        prod = s < t ? prod * g1[u] : 1.f;
+        o[u] = s <= t ? prod : 0.f;
+      }
+      *reinterpret_cast<f32x4*>(am + s0) = o;
+    }
+    float th = 1.f, apv = 1.f;
     for (int r0 = 0; r0 < cs; r0 += 4) {
       float g1[4], g2[4];
 #pragma unroll
       for (int u = 0; u < 4; ++u) { g1[u] = gt[r0 + u]; g2[u] = ga[r0 + u]; }
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
-        const int r = r0 + u;
-        th = r <= t ? th * g1[u] : th;
-        apv = r <= t ? apv * g2[u] : apv;
-        prod = r > t ? prod * g2[u] : 1.f;
-        am[(long long)r * cs] = r >= t ? prod : 0.f;
+        th = r0 + u <= t ? th * g1[u] : th;
+        apv = r0 + u <= t ? apv * g2[u] : apv;
       }
     }
     p.thp[tb * cs + t] = th;

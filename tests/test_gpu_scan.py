@@ -340,3 +340,32 @@ def test_scan_from_equals_in_place(D, E, cs, compute, n_chunks):
             bad = [L.ptr(t) for t in (*x, *gates, *st0, st0[0], *out[1:], y, tr, ws)]
             assert lib.atlas_scan_fwd_from(desc, *bad, nb, L.stream_ptr(x[0].device)) == 1   # overlapping states
     assert all(torch.equal(a, b) for a, b in zip(run["from"], run["place"]))
+
+
+@pytest.mark.parametrize("cs", [4, 64, 100, 128])
+def test_decay_table_order(cs):
+    """a(s->t) = alpha_t alpha_(t-1) .. alpha_(s+1) is multiplied in this order,
+    in fp32 (the chunk recurrence amplifies its last bit, so results that
+    stay the same need it).  Read back from the workspace of a one-chunk call,
+    where the tables lie at a multiple of 64 floats."""
+    import torch
+    from atlas_amd import _lib as L
+    g = torch.Generator(device="cuda").manual_seed(cs)
+    D = E = 32
+    x = [torch.randn(1, cs, 1, D, device="cuda", generator=g) for _ in range(3)]
+    gates = [torch.sigmoid(torch.randn(1, cs, 1, device="cuda", generator=g)) for _ in range(4)]
+    st = [torch.randn(1, 1, D, E, device="cuda", generator=g) for _ in range(4)]
+    desc = L.ScanDesc(B=1, T=cs, H=1, D=D, E=E, chunk_size=cs, omega_window=8, ns_steps=5, io_dtype=0, gate_dtype=0,
+                      compute=L.COMPUTE_F32)
+    lib, y = L.get_lib(), torch.empty_like(x[0])
+    nb = lib.atlas_scan_workspace_size(desc)
+    ws = torch.zeros(nb // 4, device="cuda")
+    L.check(lib.atlas_scan_fwd(desc, *(L.ptr(t) for t in (*x, *gates, *st, y, ws)), nb, L.stream_ptr(y.device)))
+    al = gates[0].flatten().cpu().numpy()
+    want = np.zeros((cs, cs), np.float32)
+    for t in range(cs):
+        want[t, t] = prod = np.float32(1)
+        for s in range(t - 1, -1, -1):
+            want[t, s] = prod = prod * al[s + 1]
+    flat, want = ws.cpu().numpy(), want.ravel()
+    assert any(np.array_equal(flat[o:o + cs * cs], want) for o in range(0, flat.size - cs * cs + 1, 64))
