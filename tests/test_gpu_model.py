@@ -329,7 +329,8 @@ def test_layer_prologue_mixed_dtypes(K, proj_dtype, out_dtype, T):
 
 
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16", "float16"])
-@pytest.mark.parametrize("shape", [(1, 1), (3, 7), (5, 512), (2, 3, 520), (9, 513), (1, 4104), (0, 64)])
+@pytest.mark.parametrize("shape", [(1, 1), (3, 7), (5, 512), (2, 3, 520), (9, 513), (1, 4104), (0, 64), (4, 31),
+                                   (70, 32), (6, 33), (2, 8191), (3, 8192), (2, 8193)])
 def test_rms_norm_rows(dtype, shape):
     """The fused row norm (16-byte rows, odd rows and bases, one row to several
     workgroups) against fp64: one rounding of the dtype and an fp32 sum of C
@@ -352,3 +353,50 @@ def test_rms_norm_rows(dtype, shape):
         for y in forms:
             assert y.dtype == dt and y.shape == x.shape
             assert bool(((y.double() - want).abs() <= tol * want.abs() + 2.0 ** -24).all())
+
+
+def test_rms_norm_under_modes_and_transforms():
+    """What looks into or rewrites a call finds the torch operations: function
+    and dispatch modes, forward-mode derivatives (dual tensors and torch.func),
+    tracing; a view that only carries a negation has it applied."""
+    torch = _torch()
+    import torch.autograd.forward_ad as fwd
+    from atlas_amd import rms_norm
+    from torch.fx.experimental.proxy_tensor import make_fx
+    from torch.overrides import TorchFunctionMode
+    from torch.utils._python_dispatch import TorchDispatchMode
+    g = torch.Generator(device="cuda").manual_seed(0)
+    x, t = (torch.randn(3, 64, device="cuda", generator=g) for _ in range(2))
+
+    def exact(x):
+        return x * (x.pow(2).mean(-1, keepdim=True) + 1e-6).rsqrt()
+
+    def close(a, b):
+        return float((a.double() - b).norm() / b.norm()) <= 1e-6
+
+    seen = []
+
+    class Functions(TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            seen.append(getattr(func, "__name__", ""))
+            return func(*args, **(kwargs or {}))
+
+    class Dispatch(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            seen.append(func.__name__)
+            return func(*args, **(kwargs or {}))
+
+    for mode in (Functions, Dispatch):
+        seen.clear()
+        with torch.no_grad(), mode():
+            y = rms_norm(x)
+        assert any("rsqrt" in n for n in seen), mode
+        assert close(y, exact(x.double()))
+    _, want = torch.func.jvp(exact, (x.double(),), (t.double(),))
+    with torch.no_grad(), fwd.dual_level():
+        assert close(fwd.unpack_dual(rms_norm(fwd.make_dual(x, t))).tangent, want)
+    assert close(torch.func.jvp(rms_norm, (x,), (t,))[1], want)
+    with torch.no_grad():
+        for traced in (torch.jit.trace(rms_norm, (x,)), make_fx(rms_norm)(x)):
+            assert close(traced(t), exact(t.double()))
+    assert close(rms_norm(torch._neg_view(x)), exact(-x.double()))
