@@ -236,7 +236,8 @@ def _scan_forward(q, k, v, alpha, eta, theta, gamma, state, chunk_size, omega_wi
     for name, t in (("alpha", al), ("eta", et), ("theta", th)):
         if tuple(t.shape) != (B, T, H):
             raise ValueError(f"{name} shape {tuple(t.shape)} != {(B, T, H)}")
-    st = [t.float().contiguous() for t in state]
+    # (resolve_neg: a negated view keeps only a bit through float and contiguous)
+    st = [t.float().contiguous().resolve_neg() for t in state]
     if tuple(st[0].shape) != (B, H, D, E) or tuple(st[1].shape) != (B, H, E, D):
         raise ValueError("state shapes do not match (B, H, D, E) / (B, H, E, D)")
     # the scan reads the state in 16-byte rows (a view may start anywhere)

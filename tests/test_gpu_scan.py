@@ -369,3 +369,18 @@ def test_decay_table_order(cs):
             want[t, s] = prod = prod * al[s + 1]
     flat, want = ws.cpu().numpy(), want.ravel()
     assert any(np.array_equal(flat[o:o + cs * cs], want) for o in range(0, flat.size - cs * cs + 1, 64))
+
+
+def test_scan_from_a_negated_view():
+    """An initial state that is a view with torch's negation bit set (as the
+    imaginary part of a conjugate is): the same result as from its values."""
+    import torch
+    from atlas_amd import DeepMemoryState, memory_scan
+    g = torch.Generator(device="cuda").manual_seed(0)
+    rnd = lambda *s: torch.randn(*s, device="cuda", generator=g)  # noqa: E731
+    x = [rnd(1, 70, 2, 32) * 0.3 for _ in range(3)]
+    gates = [torch.sigmoid(rnd(1, 70, 2)) for _ in range(4)]
+    st = [rnd(1, 2, 32, 64), rnd(1, 2, 64, 32), rnd(1, 2, 32, 64), rnd(1, 2, 64, 32)]
+    a, sa = memory_scan(*x, *gates, DeepMemoryState(*(torch._neg_view(t) for t in st)), 64, 8, 5)
+    b, sb = memory_scan(*x, *gates, DeepMemoryState(*(-t for t in st)), 64, 8, 5)
+    assert all(torch.equal(p, q) for p, q in zip((a, *sa), (b, *sb)))
