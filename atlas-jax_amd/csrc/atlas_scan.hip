@@ -685,15 +685,26 @@ extern "C" atlas_status atlas_scan_fwd_from(const atlas_scan_desc* d, const void
   if (s != ATLAS_OK && !generic) return s;
   const float* init[4] = {W1_init, W2_init, S1_init, S2_init};
   float* out[4] = {W1, W2, S1, S2};
-  const size_t n = (size_t)d->B * d->H * d->D * d->E;
+  const size_t n = (size_t)d->B * d->H * d->D * d->E, sb = n * sizeof(float);
+  // y's bytes where its rows follow each other without gaps (else 0: not compared)
+  const long long rs = d->x_stride_h ? d->x_stride_h : d->D, ts = d->x_stride_t ? d->x_stride_t : (long long)d->H * d->D,
+                  bs = d->x_stride_b ? d->x_stride_b : (long long)d->T * d->H * d->D;
+  const bool dense = (d->H == 1 || rs == d->D) && (d->T == 1 || ts == (long long)d->H * d->D) &&
+                     (d->B == 1 || bs == (long long)d->T * d->H * d->D);
+  const size_t yb = dense ? (size_t)d->B * d->T * d->H * d->D * (d->io_dtype == ATLAS_DTYPE_F32 ? 4 : 2) : 0;
+  const size_t tb = state_trace ? (size_t)((d->T + (long long)d->chunk_size - 1) / d->chunk_size) * 4 * sb : 0;
+  auto overlap = [](const void* p, size_t np, const void* q, size_t nq) {
+    const uintptr_t x = reinterpret_cast<uintptr_t>(p), z = reinterpret_cast<uintptr_t>(q);
+    return x < z + nq && z < x + np;
+  };
   for (int i = 0; i < 4; ++i) {
     if (!init[i] || !out[i]) return fail(ATLAS_ERR_INVALID_ARGUMENT, "NULL state pointer");
     if (misaligned16(init[i])) return fail(ATLAS_ERR_INVALID_ARGUMENT, "the initial state must be 16-byte aligned");
-    for (int j = 0; j < 4; ++j) {
-      const uintptr_t x = reinterpret_cast<uintptr_t>(init[i]), z = reinterpret_cast<uintptr_t>(out[j]);
-      if (x < z + n * sizeof(float) && z < x + n * sizeof(float))
+    for (int j = 0; j < 4; ++j)
+      if (overlap(init[i], sb, out[j], sb))
         return fail(ATLAS_ERR_INVALID_ARGUMENT, "the initial state overlaps the output state");
-    }
+    if ((yb && overlap(init[i], sb, y, yb)) || (tb && overlap(init[i], sb, state_trace, tb)))
+      return fail(ATLAS_ERR_INVALID_ARGUMENT, "the initial state overlaps y or the state trace");
   }
   if (state_trace && misaligned16(state_trace))
     return fail(ATLAS_ERR_INVALID_ARGUMENT, "state_trace must be 16-byte aligned");

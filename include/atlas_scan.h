@@ -130,7 +130,8 @@ atlas_status atlas_scan_fwd(const atlas_scan_desc* desc,
 /* atlas_scan_fwd out of place: starts from W1_init .. S2_init (only read) and
  * writes the final state to W1 .. S2, without the copies that an in-place
  * call needs to keep its initial state.  The initial arrays may overlap none
- * of the outputs.  state_trace: as in atlas_scan_fwd_trace, or NULL.  Same
+ * of the outputs (INVALID_ARGUMENT; a y with gaps between its rows is not
+ * checked).  state_trace: as in atlas_scan_fwd_trace, or NULL.  Same
  * shapes, workspace and errors as atlas_scan_fwd. */
 atlas_status atlas_scan_fwd_from(const atlas_scan_desc* desc,
                                  const void* q, const void* k, const void* v,

@@ -142,6 +142,29 @@ def test_scan_rejects_misaligned_pointers(lib):
     assert st == 1 and "workspace" in lib.atlas_last_error().decode()
 
 
+def test_scan_from_rejects_overlapping_outputs(lib):
+    """The out-of-place scan refuses, before anything is launched, an initial
+    state that shares memory with the final state, with y or with the trace:
+    their first and last bytes, on the phase kernels and the per-token path."""
+    for d in (_desc(B=1, T=100, H=2), _desc(B=1, T=100, H=2, D=48, E=96, chunk_size=6, compute=0)):
+        ws = lib.atlas_scan_workspace_size(d)
+        sb, yb = 4 * d.B * d.H * d.D * d.E, 2 * d.B * d.T * d.H * d.D
+        tb = -(-d.T // d.chunk_size) * 4 * sb
+        at = lambda x: ctypes.c_void_p(x)  # noqa: E731
+        base = 1 << 30
+        others = [at(base)] * 7
+        init, out = [2 * base + i * sb for i in range(4)], [3 * base + i * sb for i in range(4)]
+        y, tr = 4 * base, 5 * base
+        assert max(yb, tb, 4 * sb) < base
+        for i in range(4):
+            for where, size in ((out[i], sb), (y, yb), (tr, tb)):
+                for x in (where - sb + 16, where + size - 16):
+                    moved = [x if j == i else v for j, v in enumerate(init)]
+                    st = lib.atlas_scan_fwd_from(d, *others, *map(at, moved), *map(at, out), at(y), at(tr), at(6 * base),
+                                                 ws, ctypes.c_void_p(0))
+                    assert st == 1 and "overlaps" in lib.atlas_last_error().decode(), (i, where)
+
+
 def test_workspace_does_not_grow_with_sequence_length(lib):
     """The gate tables are held for a window of chunks, so the workspace
     depends on B*H, D, E and the chunk size, not on T (C2 and C4 shapes)."""
