@@ -171,14 +171,6 @@ struct ModeF32 {
   __device__ __forceinline__ static frag scale(frag f, float s) { return f * s; }
   __device__ __forceinline__ static frag scale_v(frag f, frag s) { return f * s; }
   __device__ __forceinline__ static elem to_elem(float x) { return x; }
-  __device__ __forceinline__ static frag identity(int kb, int c, int h) {
-    return (c == kslot(kb, h, 0)) ? 1.f : 0.f;
-  }
-  using afrag = float;
-  __device__ __forceinline__ static afrag a_from_c(const f32x16& t, int kb) { return t[kb]; }
-  __device__ __forceinline__ static afrag a_identity(int kb, int c, int h, float w) {
-    return (c == kslot(kb, h, 0)) ? w : 0.f;
-  }
 };
 
 // Polar-Express coefficient rows (a, b, c) of atlas_jax/memory_layer.py:34-40.

@@ -774,7 +774,9 @@ atlas_status launch_vjp(long long n, int ns, int tall, const float* X, float* G,
     if (e != hipSuccess) return fail_hip(e, "pe_vjp shared-memory attribute");
     attr_set = true;
   }
-  // the scratch holds VJP_GRID x (ns - 1) iterates: enough for PER_CU (at most 2) workgroups per slot
+  // vjp_scratch_floats holds ns - 1 iterates for each of VJP_GRID: enough for PER_CU workgroups' ns - 3 up to ns = 5
+  static_assert(V::PER_CU * V::scratch_floats(5) <= size_t(4) * D * E && V::PER_CU * V::scratch_floats(4) <= size_t(3) * D * E,
+                "scratch of the resident workgroups");
   const long long grid = std::min<long long>(n, (long long)V::PER_CU * VJP_GRID);
   hipLaunchKernelGGL((pe_vjp_split_kernel<D, E>), dim3((unsigned)grid), dim3(256), bytes, st, n, ns, tall, X, G, scratch);
   const hipError_t e = hipGetLastError();

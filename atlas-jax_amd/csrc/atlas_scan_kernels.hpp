@@ -634,7 +634,7 @@ __device__ __forceinline__ void store_rows4(const f32x4 (&v)[MAXF4], typename M:
 //   MAT == 2 (W2, first MLP layer): L2_j and h partials (hloc).
 //   MAT == 1 (W1, second layer):    h -> g for the slice, L1_j, y partials.
 // LSH: L_j accumulates in an fp32 LDS array (else in accumulator registers
-// through an identity MFMA); the LDS form needs D*E*4 more bytes of LDS.
+// by multiply-adds); the LDS form needs D*E*4 more bytes of LDS.
 // ===========================================================================
 template <class M, int D, int E, int MAT, bool LSH>
 __global__ void __launch_bounds__(NTHREADS)
@@ -646,6 +646,8 @@ phase_kernel(ScanArgs p) {
   using frag = typename M::frag;
   using LY = PhaseLayout<M, D, E>;
   static_assert(sizeof(elem) == 4, "fp32 mode (the fp16 mode runs phase16_kernel and phase_wide_kernel)");
+  static_assert(PESplit<D, E>::ELEMS * sizeof(_Float16) <= Scr<M>::template elems<D>() * sizeof(elem),
+                "Polar-Express stages its operands in the wave's scratch");
   extern __shared__ __attribute__((aligned(16))) char smem[];
   const LY L(p.cs);
 
@@ -889,9 +891,6 @@ phase_kernel(ScanArgs p) {
 
   const int tpw = ts / NW;
   const int nkb = (n + M::KB - 1) / M::KB;
-  frag idf[KPT];   // identity B operand for the fp16 read-out transpose
-#pragma unroll
-  for (int kb = 0; kb < KPT; ++kb) idf[kb] = M::identity(kb, c, h);
   for (int it = 0; it < tpw; ++it) {
     const int sl = wv * tpw + it;      // slice-local token
     const int t = tok0 + sl;           // chunk-local token
@@ -1010,37 +1009,17 @@ phase_kernel(ScanArgs p) {
             RO[J] = M::mma(M::from_c(X[K][J], kb), M::scale(load_qf(K, kb), wt), RO[J]);
     } else {
       // yloc[d][t'] += sum_e P1[d][e] g_t'[e] w(t')
-      if constexpr (LY::EB == 2) {
-        // P1 rows via the identity-product transpose: (P1 tile)^T * I in C
-        // layout has e along its rows, so as the A operand it supplies P1
-        // with the k assignment of a C-layout tile (kslot).
+      // P1 rows via the scratch transpose
+      constexpr int SP = Scr<M>::SP;
 #pragma unroll
-        for (int Je = 0; Je < TJ; ++Je) {
-          frag gw[KPT];
+      for (int Je = 0; Je < TJ; ++Je) {
+        scr_put_cols<M, TI, TJ>(X, Je, scr);
 #pragma unroll
-          for (int kb = 0; kb < KPT; ++kb) gw[kb] = M::scale(M::ld_cslot(Gs + c * LY::GSP + 32 * Je, kb, h), wt);
+        for (int kb = 0; kb < KPT; ++kb) {
+          const frag gw = M::scale(M::ld_contig(Gs + c * LY::GSP + 32 * Je, kb, h), wt);
 #pragma unroll
-          for (int Id = 0; Id < TI; ++Id) {
-            f32x16 tt = zero16();
-#pragma unroll
-            for (int kb = 0; kb < KPT; ++kb) tt = M::mma(M::from_c(X[Id][Je], kb), idf[kb], tt);
-#pragma unroll
-            for (int kb = 0; kb < KPT; ++kb) RO[Id] = M::mma(M::from_c(tt, kb), gw[kb], RO[Id]);
-          }
-        }
-      } else {
-        // P1 rows via the scratch transpose
-        constexpr int SP = Scr<M>::SP;
-#pragma unroll
-        for (int Je = 0; Je < TJ; ++Je) {
-          scr_put_cols<M, TI, TJ>(X, Je, scr);
-#pragma unroll
-          for (int kb = 0; kb < KPT; ++kb) {
-            const frag gw = M::scale(M::ld_contig(Gs + c * LY::GSP + 32 * Je, kb, h), wt);
-#pragma unroll
-            for (int Id = 0; Id < TI; ++Id)
-              RO[Id] = M::mma(M::ld_contig(scr + (32 * Id + c) * SP, kb, h), gw, RO[Id]);
-          }
+          for (int Id = 0; Id < TI; ++Id)
+            RO[Id] = M::mma(M::ld_contig(scr + (32 * Id + c) * SP, kb, h), gw, RO[Id]);
         }
       }
     }
