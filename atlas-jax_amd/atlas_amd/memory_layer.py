@@ -285,10 +285,9 @@ def rms_norm(x):
     So do rows of under 32 or over 8192 elements, one wave each in the kernel:
     a million rows of 16 take it 141 us in fp32 (torch 107; of 32: 146
     against 204), one row of 32 767 75 us (torch 25; of 8192: 8 against 24)."""
-    if (type(x) in (torch.Tensor, nn.Parameter) and x.layout == torch.strided and x.is_cuda and x.dtype in _RMS_DTYPES
-            and x.dim() > 0 and x.numel() > 0 and 32 <= x.shape[-1] <= 8192
-            and not (x.requires_grad and torch.is_grad_enabled()) and _seen_by_eager_only(x)
-            and x.is_contiguous() and not x.is_neg() and x.device.index == torch.cuda.current_device()):
+    if (type(x) in (torch.Tensor, nn.Parameter) and _seen_by_eager_only(x) and x.layout == torch.strided and x.is_cuda
+            and x.dtype in _RMS_DTYPES and x.dim() > 0 and x.numel() > 0 and 32 <= x.shape[-1] <= 8192
+            and not (x.requires_grad and torch.is_grad_enabled()) and x.is_contiguous() and not x.is_neg() and x.device.index == torch.cuda.current_device()):
         y = torch.empty_like(x)
         C = x.shape[-1]
         L.check(L.get_lib().atlas_rms_norm(x.numel() // C, C, L.ptr(x), L.ptr(y), L.dtype_code(x.dtype),
