@@ -95,9 +95,9 @@ __device__ __forceinline__ void pe_load(f32x16 (&X)[D / 32][E / 32], const void*
         }
   }
 }
-// X * ps to y, laid out as pe_load reads it
+// X to y, laid out as pe_load reads it
 template <int D, int E, int DT, int PATH>
-__device__ __forceinline__ void pe_store(const f32x16 (&X)[D / 32][E / 32], float ps, void* y, int rows, int cols, bool tall) {
+__device__ __forceinline__ void pe_store(const f32x16 (&X)[D / 32][E / 32], void* y, int rows, int cols, bool tall) {
   constexpr int TI = D / 32, TJ = E / 32;
   // (opaque: the offsets are formed again rather than kept, spilled, across
   // Polar-Express)
@@ -115,7 +115,7 @@ __device__ __forceinline__ void pe_store(const f32x16 (&X)[D / 32][E / 32], floa
           const int i = 32 * I + 8 * q + 4 * h, j = 32 * J + c;
           if (i < rows && j < cols)
             *reinterpret_cast<f32x4*>(static_cast<float*>(y) + j * rows + i) =
-                f32x4{X[I][J][4 * q] * ps, X[I][J][4 * q + 1] * ps, X[I][J][4 * q + 2] * ps, X[I][J][4 * q + 3] * ps};
+                f32x4{X[I][J][4 * q], X[I][J][4 * q + 1], X[I][J][4 * q + 2], X[I][J][4 * q + 3]};
         }
     } else if constexpr (PATH == PE_WIDEV) {
       typedef typename PEVec<TJ>::type vec;
@@ -124,7 +124,7 @@ __device__ __forceinline__ void pe_store(const f32x16 (&X)[D / 32][E / 32], floa
         const int i = 32 * I + crow(r, h), j = TJ * c;
         vec v;
 #pragma unroll
-        for (int J = 0; J < TJ; ++J) v[J] = X[I][J][r] * ps;
+        for (int J = 0; J < TJ; ++J) v[J] = X[I][J][r];
         if (i < rows && j < cols) *reinterpret_cast<vec*>(static_cast<float*>(y) + i * cols + j) = v;
       }
     } else {
@@ -133,7 +133,7 @@ __device__ __forceinline__ void pe_store(const f32x16 (&X)[D / 32][E / 32], floa
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
           const int i = 32 * I + crow(r, h), j = 32 * J + c;
-          if (i < rows && j < cols) pe_st1<DT>(y, i * si + j * sj, X[I][J][r] * ps);
+          if (i < rows && j < cols) pe_st1<DT>(y, i * si + j * sj, X[I][J][r]);
         }
     }
   }
@@ -162,8 +162,8 @@ pe_split_kernel(long long n, int d1, int d2, int ns, float eps, const void* X, v
   const long long base = mat * (long long)d1 * d2 * (DT == 0 ? 4 : 2);
   f32x16 Xr[TI][TJ];
   pe_load<D, E, DT, PATH>(Xr, static_cast<const char*>(X) + base, rows, cols, tall);
-  const float ps = polar_express_wave_split<D, E>(Xr, ns, eps, xs_all + w * PESplit<D, E>::ELEMS);
-  pe_store<D, E, DT, PATH>(Xr, ps, static_cast<char*>(Y) + base, rows, cols, tall);
+  polar_express_wave_split<D, E>(Xr, ns, eps, xs_all + w * PESplit<D, E>::ELEMS);
+  pe_store<D, E, DT, PATH>(Xr, static_cast<char*>(Y) + base, rows, cols, tall);
 }
 
 // fp16 operands, wide side <= 128: the scan's own Polar-Express
@@ -347,8 +347,9 @@ pe_pair_kernel(long long n, int d1, int d2, int ns, float eps, const void* X, vo
 //   B     = b G + c G^2, the same tiles, shared the same way;
 //   X     <- a X + B X for the wave's column block.
 // Every sum has a fixed order (bitwise reproducible).  2 048 matrices of 96 x
-// 192, 5 steps: 356 us (1019 us on fp32 operands, staged a block at a time
-// with all nine Gram tiles).
+// 192, 5 steps: 317 us a call (369 us with one scale for all columns, at three
+// waves per SIMD instead of four; 1019 us on fp32 operands, staged a block at a
+// time with all nine Gram tiles).
 template <int TI, int NW>
 struct PEWg {
   static constexpr int DP = 32 * TI;
@@ -512,17 +513,20 @@ pe_wg_kernel(long long n, int d1, int d2, int ns, float eps, const void* X, void
       f32x16 acc[TI];
 #pragma unroll
       for (int I = 0; I < TI; ++I) acc[I] = zero16();
+      // the column's largest entry to [2^12, 2^13) (columns far below the others keep their bits)
+      const int ke = column_exponent<TI>(Xr, 13);
+      const float sc = __builtin_amdgcn_ldexpf(1.f, ke);
 #pragma unroll
       for (int K = 0; K < TI; ++K)
 #pragma unroll
         for (int kb = 0; kb < 2; ++kb) {
-          const SFrag x = split_c(Xr[K], kb, XS);
+          const SFrag x = split_c(Xr[K], kb, sc);
 #pragma unroll
           for (int I = 0; I < TI; ++I) acc[I] = mma_split(get_frag(slot(fB, K, I, kb)), x, acc[I]);
           __builtin_amdgcn_sched_barrier(0);   // keeps later fragments' loads from being hoisted (registers)
         }
 #pragma unroll
-      for (int I = 0; I < TI; ++I) Xr[I] = pa * Xr[I] + acc[I] * (1.f / (BS * XS));
+      for (int I = 0; I < TI; ++I) Xr[I] = pa * Xr[I] + acc[I] * __builtin_amdgcn_ldexpf(1.f / BS, -ke);
     }
     __syncthreads();   // B has been read: the blocks may be staged over it
   }

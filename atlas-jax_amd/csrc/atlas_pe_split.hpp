@@ -3,7 +3,14 @@
 //
 // An fp32 operand x, scaled by a power of two into fp16's range, is held as
 // two fp16 numbers, hi = fp16(s x) and lo = fp16(s x - hi): together 22 to 23
-// significant bits.  A product takes three MFMAs with fp32 accumulation,
+// significant bits while s x is above 2^-3 (lo ends at fp16's 2^-24), one less
+// for each power of two below that, none under 2^-25.  With the largest at 2^12
+// to 2^15 that is about 2^-16 of it.  So the columns (the longer side) of
+// Polar-Express and its VJP carry scales of their own, at any size down to 2^-60
+// of the largest; rows share their matrix's scale: a row's result keeps fp32's
+// relative accuracy while the row is above about 2^-20 of the largest (the steps
+// lift it), and is accurate relative to the matrix below that.
+// A product takes three MFMAs with fp32 accumulation,
 // lo hi + hi lo + hi hi (the dropped lo lo is below 2^-24 of the operands'
 // product).  Each v_mfma_f32_32x32x16_f16 adds 16 exact products to the fp32
 // accumulator where v_mfma_f32_32x32x2f32 rounds after every two, so the sums
@@ -52,17 +59,36 @@ __device__ __forceinline__ f32x16 mma_split(const SFrag& a, const SFrag& b, f32x
   return ModeF16::mma(a.hi, b.hi, c);
 }
 
+// k with 2^k times the largest entry of this lane's column (TI C-layout tiles)
+// in [2^(top - 1), 2^top), at most 100 + top (a column of zeros: top).
+template <int TI>
+__device__ __forceinline__ int column_exponent(const f32x16 (&t)[TI], int top) {
+  float m = 0.f;
+#pragma unroll
+  for (int I = 0; I < TI; ++I)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) m = fmaxf(m, fabsf(t[I][r]));
+  float m0, m1;
+  swap32(m, m0, m1);   // the other rows lie in the other half
+  return top + min(-__builtin_amdgcn_frexp_expf(fmaxf(m0, m1)), 100);
+}
+
 // Per-step factors of the split Polar-Express.  The iterate is carried as
 // X_s = mu X, mu_0 = 2^30, mu <- mu / a each step (so the step needs no a X
 // multiply, as in polar_express_wave_t).  Its operand is x = sx X_s, the Gram
 // accumulates nu^2 G (nu = sx mu), its operand is g = sg nu^2 G = gamma G; then
 //   R = gamma^2 (G^2 + (b/c) G)   accumulated onto kappa (nu^2 G),
-//   r = rho R = (B / a) / sx      the update's operand: X_s <- X_s + r x.
+//   r = rho R = 2^15 (B / a)      an operand of the update X_s <- X_s + r (2^-15 X_s).
 // All scales are powers of two chosen so that every operand's largest entry
-// (|X|, |G|^(1/2) <= 2, |B / a| <= 1 over the iteration) stays below 2^15.
+// (|X|, |G|^(1/2) <= 2, |B / a| <= 1 over the iteration) stays below 2^15 (r: at
+// most 2^15).  Each column of X_s is carried times a power of two 2^k of its own
+// (its largest entry 2^26 to 2^27 at first, so that its norm, which the steps do not
+// increase, stays below 2^30): the update works on columns, so a column far below
+// the others keeps its bits; only the Gram's operands are scaled back by 2^-k.
 struct PEScale {
   float sx, sg, kappa, rho;
 };
+constexpr float PE_XU = 1.f / 32768.f;   // X_s as the update's operand
 constexpr double kPEd64[5][3] = {
     {8.156554524902461, -22.48329292557795, 15.878769915207462},
     {4.042929935166739, -2.808917465908714, 0.5000178451051316},
@@ -77,7 +103,7 @@ constexpr PEScale pe_scale(int st) {
   double sg = 1.0;
   while (sg * nu * nu > 4096.0) sg *= 0.5;                    // gamma in (2^11, 2^12]
   const double gamma = sg * nu * nu, a = kPEd64[st][0], b = kPEd64[st][1], c = kPEd64[st][2];
-  return {(float)sx, (float)sg, (float)(b / c * gamma * gamma / (nu * nu)), (float)(c / (a * gamma * gamma * sx))};
+  return {(float)sx, (float)sg, (float)(b / c * gamma * gamma / (nu * nu)), (float)(32768.0 * c / (a * gamma * gamma))};
 }
 __constant__ static const PEScale kPEsplit[5] = {pe_scale(0), pe_scale(1), pe_scale(2), pe_scale(3), pe_scale(4)};
 __constant__ static const float kPEmu[6] = {(float)(1.0 / pe_mu(0)), (float)(1.0 / pe_mu(1)), (float)(1.0 / pe_mu(2)),
@@ -152,11 +178,14 @@ struct PESplit {
     return {tr2(p, p8), tr2(p + BLOCK, p8 + BLOCK)};
   }
 
+  // exponent k of this lane's column of block J (ke: four signed bytes)
+  __device__ __forceinline__ static int column_exp(int ke, int J) { return (ke << (24 - 8 * J)) >> 24; }
+
   // nu^2 G, upper tiles (I, I2 >= I)
-  __device__ __forceinline__ static void gram(const f32x16 (&X)[TI][TJ], f32x16 (&A)[TI][TI], float sx, _Float16* xs) {
+  __device__ __forceinline__ static void gram(const f32x16 (&X)[TI][TJ], f32x16 (&A)[TI][TI], float sx, int ke, _Float16* xs) {
 #pragma unroll
     for (int J = 0; J < TJ; ++J) {
-      put_block(X, J, sx, xs);
+      put_block(X, J, __builtin_amdgcn_ldexpf(sx, -column_exp(ke, J)), xs);
       SFrag th[TI][2];
 #pragma unroll
       for (int I = 0; I < TI; ++I)
@@ -213,7 +242,7 @@ struct PESplit {
       for (int K = 0; K < TI; ++K) {
         asm volatile("" : "+v"(X[K][J]));   // split again rather than kept from the Gram's staging (registers)
 #pragma unroll
-        for (int kb = 0; kb < 2; ++kb) xf[K][kb] = split_c(X[K][J], kb, k.sx);
+        for (int kb = 0; kb < 2; ++kb) xf[K][kb] = split_c(X[K][J], kb, PE_XU);
       }
 #pragma unroll
       for (int K = 0; K < TI; ++K)
@@ -225,12 +254,11 @@ struct PESplit {
   }
 };
 
-// One matrix per wave, fp32 accuracy.  X is left as X_s; returns the factor
-// that turns it into PolarExpress(X).
+// One matrix per wave, fp32 accuracy: X <- PolarExpress(X).
 template <int D, int E>
-__device__ __forceinline__ float polar_express_wave_split(f32x16 (&X)[D / 32][E / 32], int ns, float norm_eps,
-                                                          _Float16* xs) {
+__device__ __forceinline__ void polar_express_wave_split(f32x16 (&X)[D / 32][E / 32], int ns, float norm_eps, _Float16* xs) {
   using P = PESplit<D, E>;
+  static_assert(D <= 64 && E <= 128, "column norms, packed exponents");
   float ss = 0.f;
 #pragma unroll
   for (int I = 0; I < P::TI; ++I)
@@ -240,17 +268,39 @@ __device__ __forceinline__ float polar_express_wave_split(f32x16 (&X)[D / 32][E 
       for (int r = 0; r < 16; ++r) ss += X[I][J][r] * X[I][J][r];
   ss = wave_sum(ss);
   const float s = 1.f / (sqrtf(ss + norm_eps) * 1.01f + 1e-6f);
+  int ke = 0;
 #pragma unroll
-  for (int I = 0; I < P::TI; ++I)
+  for (int J = 0; J < P::TJ; ++J) {
+    float m = 0.f;
 #pragma unroll
-    for (int J = 0; J < P::TJ; ++J) X[I][J] = X[I][J] * s * 1073741824.f;   // mu_0 = 2^30
+    for (int I = 0; I < P::TI; ++I)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        X[I][J][r] *= s;
+        m = fmaxf(m, fabsf(X[I][J][r]));
+      }
+    float m0, m1;
+    swap32(m, m0, m1);   // the column's other rows
+    // 2^k m in [2^-4, 2^-3): the column's norm is below sqrt(D) / 8 <= 1 (a column of zeros: k = -3)
+    const int k = min(-3 - __builtin_amdgcn_frexp_expf(fmaxf(m0, m1)), 90);
+    ke |= (k & 255) << (8 * J);
+#pragma unroll
+    for (int I = 0; I < P::TI; ++I)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) X[I][J][r] = __builtin_amdgcn_ldexpf(X[I][J][r], 30 + k);   // mu_0 = 2^30
+  }
   for (int st = 0; st < ns; ++st) {
     const PEScale k = kPEsplit[st];
     f32x16 A[P::TI][P::TI];
-    P::gram(X, A, k.sx, xs);
+    P::gram(X, A, k.sx, ke, xs);
     P::apply(X, A, k, xs);
   }
-  return kPEmu[ns];
+#pragma unroll
+  for (int J = 0; J < P::TJ; ++J) {
+    const float ps = __builtin_amdgcn_ldexpf(kPEmu[ns], -P::column_exp(ke, J));
+#pragma unroll
+    for (int I = 0; I < P::TI; ++I) X[I][J] *= ps;
+  }
 }
 
 }  // namespace atlas

@@ -18,15 +18,19 @@
 //      C tiles are the B operands as they are.
 // The forward recompute has the same phases with one upper tile of A and B per
 // wave.  G is brought to a largest entry in [1, 2) by a power of two before the
-// first step and back after the normalisation (cotangents of any size,
-// subnormal ones included), and again for each step's operands; with |Y| <= 2 (|A| <= 4, |Gs| <= 1024, |C| < 2^15 for the sizes
-// compiled) fixed powers of two keep every operand in fp16's range.
+// first step and back after the normalisation (cotangents of any size, subnormal
+// ones included).  As operands, Y and G staged for the Gram-like products and A
+// and B have fixed scales (|Y| <= 2, |A| <= 4, |B| <= 8; G's is set again for each
+// step), Gs and C the ones that the largest entry of Gs allows, and the columns of
+// Y and G that B and C act on one each, so that columns far below the others keep
+// their bits (rows down to about 2^-20 of the largest do).
 // Y_1 .. Y_{ns-3} go to the workgroup's global scratch, Y_{ns-2} stays in
 // registers, Y_0 is X / nrm again.
 //
-// 4 096 matrices of 64 x 128, 5 steps: 2908 -> 640 us against fp32 MFMA on
+// 4 096 matrices of 64 x 128, 5 steps: 2908 -> 650 us against fp32 MFMA on
 // element-wise LDS operands (one workgroup per CU; the split tiles leave room
-// for two), 2 048 of 64 x 256: 7.2 -> 0.79 ms.  About 1000 products of 32
+// for two), 2 048 of 64 x 256: 7.2 -> 0.85 ms (one scale for all columns and
+// fixed ones for Gs and C: 640 us, 0.79 ms, with the small columns' bits lost).  About 1000 products of 32
 // cycles per SIMD and matrix; the barriers between the phases, with waves idle
 // where a phase has fewer tiles than waves, bound it.  Addresses and fragments
 // are kept from being hoisted (opaque lanes, fences): hoisted, 244 registers
@@ -70,7 +74,6 @@ pe_vjp_split_kernel(long long n, int ns, int tall, const float* X, float* G, flo
   constexpr float YS = 4096.f, GS = 2048.f;   // scales of Y and of G with its largest entry in [1, 2)
   constexpr float AS = 2048.f;                // A (entries <= 4) as an operand: 2^11
   constexpr float BS = 4096.f;                // B (<= 8): 2^12
-  constexpr float SS = 32.f, CS = 2.f;        // Gs (<= 1024): 2^5; C (< 2^15): 2^1
   extern __shared__ __attribute__((aligned(16))) _Float16 lds[];
   _Float16* yst = lds;                        // staged Y blocks
   _Float16* gst = lds + NB * V::BLK;          // staged G blocks
@@ -277,17 +280,19 @@ pe_vjp_split_kernel(long long n, int ns, int tall, const float* X, float* G, flo
           f32x16 acc[TI];
 #pragma unroll
           for (int I = 0; I < TI; ++I) acc[I] = zero16();
+          const int ey = column_exponent<TI>(Yp[q], 12);
+          const float ys = __builtin_amdgcn_ldexpf(1.f, ey);
 #pragma unroll
           for (int K = 0; K < TI; ++K)
 #pragma unroll
             for (int kb = 0; kb < 2; ++kb) {
-              const SFrag y = split_c(Yp[q][K], kb, YS);
+              const SFrag y = split_c(Yp[q][K], kb, ys);
 #pragma unroll
               for (int I = 0; I < TI; ++I) acc[I] = mma_split(get_frag(fB, K, I, kb), y, acc[I]);
               PE_FENCE();
             }
 #pragma unroll
-          for (int I = 0; I < TI; ++I) Y[q][I] = ka * Yp[q][I] + acc[I] * (1.f / (BS * YS));
+          for (int I = 0; I < TI; ++I) Y[q][I] = ka * Yp[q][I] + acc[I] * __builtin_amdgcn_ldexpf(1.f / BS, -ey);
         }
       __syncthreads();   // B has been read: the blocks may be staged over it
     }
@@ -337,8 +342,23 @@ pe_vjp_split_kernel(long long n, int ns, int tall, const float* X, float* G, flo
         gram_tiles(A, 0);
       } else if (w <= NT) {
         S = gs_tile(tI(w - 1), tI2(w - 1));
+        S *= 1.f / (GS * YS);   // Gs of sg G
+      }
+      {
+        float gm = 0.f;
+        if (w != 0 && w <= NT) {
+#pragma unroll
+          for (int r = 0; r < 16; ++r) gm = fmaxf(gm, fabsf(S[r]));
+        }
+        gm = wave_max(gm);
+        if (lane == 0) red[12 + w] = gm;
       }
       __syncthreads();   // the staged blocks have been read
+      // Gs as an operand: its largest entry to [2^13, 2^14); C at most 2^9 (first
+      // step: |A| <= 1, |b| + 2 |c| sqrt(D) |A| < 2^9) or 2^6 times that of Gs
+      const float SS = __builtin_amdgcn_ldexpf(
+          1.f, min(14 - __builtin_amdgcn_frexp_expf(fmaxf(fmaxf(red[12], red[13]), fmaxf(red[14], red[15]))), 24));
+      const float CS = SS * (k == 0 ? 1.f / 256.f : 1.f / 32.f);
       if (w == 0) {
 #pragma unroll
         for (int j = 0; j < NT; ++j) {
@@ -346,7 +366,6 @@ pe_vjp_split_kernel(long long n, int ns, int tall, const float* X, float* G, flo
           share(fA, A[j], tI(j), tI2(j), AS);
         }
       } else if (w <= NT) {
-        S *= 1.f / (GS * YS);   // Gs of sg G
         share(fG, S, tI(w - 1), tI2(w - 1), SS);
       }
       __syncthreads();
@@ -360,7 +379,7 @@ pe_vjp_split_kernel(long long n, int ns, int tall, const float* X, float* G, flo
       } else if (w <= NT) {
         f32x16 t = dd_tile(fG, fA, tI(w - 1), tI2(w - 1), zero16());
         t = dd_tile(fA, fG, tI(w - 1), tI2(w - 1), t);
-        S = kb_ * S + (kc / (AS * SS)) * t;
+        S = kb_ * S + kc / (AS * SS) * t;
         share(fC, S, tI(w - 1), tI2(w - 1), CS);
       }
       __syncthreads();
@@ -370,27 +389,31 @@ pe_vjp_split_kernel(long long n, int ns, int tall, const float* X, float* G, flo
           f32x16 acc[TI];
 #pragma unroll
           for (int I = 0; I < TI; ++I) acc[I] = zero16();
+          // (exponents of columns 60 or more powers of two down are held there: the factor between the sums stays finite)
+          const int eg_ = min(column_exponent<TI>(Gb[q], 12), 72), ey = min(column_exponent<TI>(Y[q], 12), 72);
+          const float gs = __builtin_amdgcn_ldexpf(1.f, eg_), ys = __builtin_amdgcn_ldexpf(1.f, ey);
 #pragma unroll
           for (int K = 0; K < TI; ++K)
 #pragma unroll
             for (int kb = 0; kb < 2; ++kb) {
-              const SFrag g = split_c(Gb[q][K], kb, sg * GS);
+              const SFrag g = split_c(Gb[q][K], kb, gs);
 #pragma unroll
               for (int I = 0; I < TI; ++I) acc[I] = mma_split(get_frag(fB, K, I, kb), g, acc[I]);
               PE_FENCE();
             }
+          const float bc = __builtin_amdgcn_ldexpf(sg * CS * (1.f / BS), ey - eg_);   // B G and C Y on one scale
 #pragma unroll
-          for (int I = 0; I < TI; ++I) acc[I] *= CS * YS / (BS * GS);   // B G and C Y on one scale
+          for (int I = 0; I < TI; ++I) acc[I] *= bc;
 #pragma unroll
           for (int K = 0; K < TI; ++K)
 #pragma unroll
             for (int kb = 0; kb < 2; ++kb) {
-              const SFrag y = split_c(Y[q][K], kb, YS);
+              const SFrag y = split_c(Y[q][K], kb, ys);
 #pragma unroll
               for (int I = 0; I < TI; ++I) acc[I] = mma_split(get_frag(fC, K, I, kb), y, acc[I]);
               PE_FENCE();
             }
-          const float ss_ = isg * (1.f / (CS * YS));
+          const float ss_ = __builtin_amdgcn_ldexpf(isg / CS, -ey);
 #pragma unroll
           for (int I = 0; I < TI; ++I) Gb[q][I] = ka * Gb[q][I] + acc[I] * ss_;
         }

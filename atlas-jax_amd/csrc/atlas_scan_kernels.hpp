@@ -957,13 +957,7 @@ phase_kernel(ScanArgs p) {
     // (on operands as two fp16 numbers, its staging in the scratch: at 64 x 128 a
     // launch of 256 workgroups with four tokens per wave takes half the time of
     // the step on fp32 MFMA)
-    {
-      const float ps = polar_express_wave_split<D, E>(X, p.ns, 1e-12f, reinterpret_cast<_Float16*>(scr));
-#pragma unroll
-      for (int I = 0; I < TI; ++I)
-#pragma unroll
-        for (int J = 0; J < TJ; ++J) X[I][J] *= ps;
-    }
+    polar_express_wave_split<D, E>(X, p.ns, 1e-12f, reinterpret_cast<_Float16*>(scr));
 
     // memory-scan partial L += a(s->end_j) P and the slice read-out partial.
     const float aend = ass[sl * ts + ts - 1];

@@ -70,7 +70,11 @@ typedef enum {
 
 /* Arithmetic of the matrix-core work inside the scan.
  *   ATLAS_COMPUTE_F32: fp32 accuracy (parity mode, ~1e-6 per chunk): fp32 MFMA,
- *     and Polar-Express on fp32 operands split into two scaled fp16 parts.
+ *     and Polar-Express on fp32 operands split into two scaled fp16 parts.  Each
+ *     line along a matrix's longer side has a scale of its own (relative accuracy
+ *     of every such line down to 2^-60 of the largest); a line along the shorter
+ *     side keeps its relative accuracy down to about 2^-20 of the largest, and is
+ *     accurate relative to the whole matrix below that.
  *   ATLAS_COMPUTE_F16: inner-gradient GEMMs in fp32 MFMA; momentum assembly,
  *     Polar-Express and read-out products with fp16 MFMA operands, fp32
  *     accumulation and fp32 master copies (~2e-3 per chunk). */

@@ -323,3 +323,51 @@ def test_pe_vjp_f32_cotangent_range(d1, d2, exp):
     err = (got.double() * 2.0 ** -exp - unit).abs().max()
     print(f"VJP {d1}x{d2} G 2^{exp}: largest error {float(err):.2e}, half a unit {2.0 ** (-150 - exp):.2e}", flush=True)
     assert err <= 2.0 ** (-150 - exp)
+
+
+@pytest.mark.parametrize("d1,d2", [(64, 128), (128, 64), (64, 64), (33, 90), (32, 32), (32, 128), (96, 192), (128, 128),
+                                   (70, 100), (64, 256), (256, 64)])
+@pytest.mark.parametrize("side,span", [("long", 40), ("long", 55), ("short", 20)])
+def test_pe_fp32_split_graded(d1, d2, side, span):
+    """Lines far below the others (columns of saturated channels): with the
+    lines along one side scaled by 2^0 to 2^-span, the worst relative error of
+    any single line, of Polar-Express and (shapes compiled) of its VJP with
+    cotangents graded alike, stays within four times that of the same
+    arithmetic in fp32 torch.  The longer side's lines have scales of their
+    own; the shorter side's share fp16's range, which holds their 22 bits down
+    to about 2^-20."""
+    torch = _torch()
+    from atlas_amd import POLAR_EXPRESS_COEFFS, polar_express
+    from atlas_amd.autograd import polar_express_vjp
+    g = torch.Generator(device="cuda").manual_seed(d1 * 257 + d2 + span)
+    n, wide = 16, d1 <= d2
+    last = (side == "long") == wide   # the graded lines are the columns of the array as it lies
+    scale = torch.exp2(-span * torch.rand(n, d2 if last else d1, device="cuda", generator=g))
+    scale = scale[:, None, :] if last else scale[:, :, None]
+    X, C = (torch.randn(n, d1, d2, device="cuda", generator=g) * scale for _ in range(2))
+
+    def plain(x):
+        x = x / (torch.sqrt((x * x).sum((-2, -1), keepdim=True) + 1e-12) * 1.01 + 1e-6)
+        for a, b, c in POLAR_EXPRESS_COEFFS:
+            A = x @ x.mT.contiguous() if wide else x.mT.contiguous() @ x
+            B = b * A + c * (A @ A)
+            x = a * x + (B @ x if wide else x @ B)
+        return x
+
+    def vjp(x, c):
+        x = x.clone().requires_grad_(True)
+        return torch.autograd.grad(plain(x), x, c)[0]
+
+    def worst(y, ref):
+        dim = -2 if last else -1
+        return float(((y.double() - ref).norm(dim=dim) / ref.norm(dim=dim)).max())
+
+    ref = plain(X.double())
+    e, bar = worst(polar_express(X, 5, precision="f32"), ref), 4 * worst(plain(X), ref)
+    print(f"graded PE {d1}x{d2} {side} 2^-{span}: {e:.2e} (bar {bar:.2e})", flush=True)
+    assert e <= bar
+    if min(d1, d2) in (32, 64) and max(d1, d2) in (32, 64, 128, 256) and (min(d1, d2), max(d1, d2)) != (32, 256):
+        ref = vjp(X.double(), C.double())
+        e, bar = worst(polar_express_vjp(X, C, 5), ref), 4 * worst(vjp(X, C), ref)
+        print(f"graded VJP {d1}x{d2} {side} 2^-{span}: {e:.2e} (bar {bar:.2e})", flush=True)
+        assert e <= bar
