@@ -660,15 +660,17 @@ __global__ void __launch_bounds__(256) prologue_bwd_reduce_kernel(const float* p
 }
 
 // (up to 69 KiB of LDS, at 256 threads to a group and four taps: the limit is
-// raised as for every launch that may pass 64 KiB)
+// raised as for every launch that passes 64 KiB)
 template <int K>
 hipError_t launch_prologue_bwd(const ProBwdArgs& a, unsigned nblk, int gthr, int nthr, bool aligned, hipStream_t st) {
   const int G = std::min(512 / gthr, PRO_BR / 4);
   const size_t lds = (size_t)gthr * (12 * K + 12 + 9) * sizeof(float);
   auto go = [&](void (*k)(ProBwdArgs, int, int, int)) {
-    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(k),
-                                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    if (e != hipSuccess) return e;
+    if (lds > 64 * 1024) {
+      const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(k),
+                                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+      if (e != hipSuccess) return e;
+    }
     hipLaunchKernelGGL(k, dim3(nblk), dim3(G * gthr), lds, st, a, nthr, gthr, G);
     return hipGetLastError();
   };
