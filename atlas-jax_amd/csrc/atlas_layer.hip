@@ -235,8 +235,8 @@ struct Poly {
 // token's row while this one is computed; q, k, v are stored 4 channels per
 // store.  The RMS norms reduce over the D/4 threads of a head on the VALU.
 // Bound by the serial chain of a run's tokens where there are few and by
-// memory where there are many: B8 T4096 H8 D64, bf16, 91 -> 61 us (205 MB,
-// 3.4 TB/s), one row of 60 tokens 49 -> 7.5 us.  Runs of 16 tokens load a
+// memory where there are many: B8 T4096 H8 D64, bf16, 91 -> 61 us (209 MB needed,
+// 3.4 TB/s; 289 MB moved, the rows before each run again), one row of 60 tokens 49 -> 7.5 us.  Runs of 16 tokens load a
 // fifth less and take 59 us and 22 us, H12 117 us against 101.
 constexpr int PRO_TT = 4;    // tokens per block
 

@@ -193,9 +193,9 @@ __device__ __forceinline__ void load_frags(const SwaArgs& a, const void* x, long
 // Bound by the VALU: per 32 queries x 64 keys and wave about 200 instructions
 // (four per score: multiply-add, exp, sum, half a conversion and half a
 // maximum; 32 exps at a quarter of the rate; the rotation and conversion of the
-// staged keys) against 16 products, 63 % VALU-busy and 26 % MFMA-busy at a
-// clock of 1.9 GHz (power).  B4 T16384 H12, window 2048, bf16: 654 us, 0.63
-// PFLOP/s; 1853 us when every block was loaded, rotated, transposed with 2-byte
+// staged keys) against 16 products, and by the latency between the two kinds:
+// 47 % VALU-busy and 24 % MFMA-busy at a clock of 1.95 GHz (power).  B4 T16384
+// H12, window 2048, bf16: 650 us, 0.63 PFLOP/s; 1853 us when every block was loaded, rotated, transposed with 2-byte
 // LDS writes and used between two barriers, 128 queries to a workgroup.  A
 // wave per SIMD more (four, spilling 19-35 registers) takes 905-1320 us, 32
 // keys to a softmax update 742 us.
@@ -460,7 +460,7 @@ __device__ __forceinline__ void store_unrot(const SwaArgs& f, void* dst, long lo
 // directly the B operands of dV^T = dO^T P and dK^T = Q^T dS (contraction over
 // queries); one copy of the q' and dO rows serves both kinds of products
 // (contiguous and transposing reads).  Bound by the VALU and the staging like
-// the forward.  B4 T4001 H12, window 2048: 305 us (642 us single-buffered, with
+// the forward.  B4 T4001 H12, window 2048: 285-305 us (642 us single-buffered, with
 // a second, transposed copy of both operands written half by half);
 // swa_bwd_q_kernel 219 us (353), swa_bwd_delta_kernel 11 us (54 with one
 // thread per row).  Twice the keys (queries) to a workgroup: no gain.
