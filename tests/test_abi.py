@@ -233,8 +233,8 @@ def test_pe_vjp_argument_checks(lib):
     one = ctypes.c_void_p(256)
     need = lib.atlas_pe_vjp_workspace_size(64, 128, 5)
     assert need > 0 and need == lib.atlas_pe_vjp_workspace_size(128, 64, 5)
-    # 64 x 256 in either mode (the fp32 kernel also keeps the iterate and the
-    # cotangent in its scratch); 32 x 256 and ns 6: not built
+    # 64 x 256 in either mode (the size callers have: room for the iterates and
+    # two further arrays); 32 x 256 and ns 6: not built
     wide = lib.atlas_pe_vjp_workspace_size(64, 256, 5)
     assert wide > 2 * need and lib.atlas_pe_vjp_workspace_size(64, 128, 6) == 0
     assert lib.atlas_pe_vjp_workspace_size(32, 256, 5) == 0
