@@ -189,9 +189,20 @@ __device__ __forceinline__ void put4(void* p, int64_t i, int dtype, f32x4 x) {
 #pragma unroll
     for (int u = 0; u < 4; ++u) store_any(p, i + u, dtype, x[u]);
 }
-// sum over the QD = 4, 8 or 16 consecutive lanes of a head
+// Sum over the QD = 4, 8 or 16 consecutive lanes of a head, the far lanes first
+// (i ^ 8, i ^ 4, i ^ 2, i ^ 1: the order fixes the last bit, and with it the
+// rounding of the 16-bit outputs).  Rotations of the row of 16 reach those
+// partners: after i ^ 8 the values repeat every 8 lanes, and so on.
 __device__ __forceinline__ float head_sum(float x, int QD) {
-  return QD == 16 ? group_sum<16>(x) : QD == 8 ? group_sum<8>(x) : group_sum<4>(x);
+  if (QD == 16) {
+    x += dpp_f<0x128>(x);
+    x += dpp_f<0x124>(x);
+    x += dpp_f<0x122>(x);
+    return x + dpp_f<0x121>(x);
+  }
+  if (QD == 8) x += dpp_f<0x1B>(dpp_f<0x141>(x));   // i ^ 7, then i ^ 3
+  x += dpp_f<0x4E>(x);
+  return x + dpp_f<0xB1>(x);
 }
 __device__ __forceinline__ float dot4(f32x4 p, f32x4 q) { return (p[0] * q[0] + p[1] * q[1]) + (p[2] * q[2] + p[3] * q[3]); }
 // the polynomial's coefficients in registers

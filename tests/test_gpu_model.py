@@ -330,6 +330,33 @@ def test_layer_prologue_mixed_dtypes(K, proj_dtype, out_dtype, T):
         assert float((a.double() - b.double()).norm() / b.double().norm()) <= (one if i < 3 else 1e-5), i
 
 
+@pytest.mark.parametrize("H,D", [(16, 16), (8, 32), (4, 64)])
+def test_layer_prologue_norm_order(H, D):
+    """The head norms add the far lanes first (i ^ D/8, .., i ^ 2, i ^ 1 of the
+    D/4 lanes with four channels each): the order decides the last bit, and
+    with it the 16-bit rounding of q and k.  A square of 2^24 or more in lane
+    0 absorbs a single 1 but not the 2 that lanes 1 and D/8 + 1 make when
+    they are added first; the same sum in any order comes from lane 0 alone."""
+    torch = _torch()
+    from atlas_amd.memory_layer import _layer_prologue_hip
+    T, HD = 96, H * D
+    big = torch.arange(4096, 4096 + 2 * T * H, 2, device="cuda")[:T * H].remainder(5790 - 4096) // 2 * 2 + 4096
+    cw = torch.zeros(3, HD, 4, device="cuda")
+    cw[..., 3] = 1
+    cb, gb = torch.zeros(3, HD, device="cuda"), torch.zeros(4, H, device="cuda")
+    out = {}
+    for name, ones in (("far first", (4, D // 2 + 4)), ("any order", (2, 3)), ("absorbed", ())):
+        x = torch.zeros(T, H, D, device="cuda")
+        x[:, :, 0] = big.view(T, H).float()
+        for c in ones:
+            x[:, :, c] = 1
+        proj = torch.cat([x.view(T, HD)] * 3 + [torch.zeros(T, 5 * H, device="cuda")], 1).contiguous()
+        q, k, *_ = _layer_prologue_hip(proj, cw, cb, None, gb, (1, T, H, D, 4, 0, 4, True, 0.1, torch.float32))
+        out[name] = torch.stack([q[..., 0], k[..., 0]])
+    assert not torch.equal(out["any order"], out["absorbed"])
+    assert torch.equal(out["far first"], out["any order"])
+
+
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16", "float16"])
 @pytest.mark.parametrize("shape", [(1, 1), (3, 7), (5, 512), (2, 3, 520), (9, 513), (1, 4104), (0, 64), (4, 31),
                                    (70, 32), (6, 33), (2, 8191), (3, 8192), (2, 8193)])
